@@ -2280,6 +2280,273 @@ __global__ __launch_bounds__(64 * kBinWaves) void pa_fp8_bin_kernel(
   }
 }
 
+// ============================================================================
+// Split decode: every (sequence, kv head) over a few workgroups, one launch
+// ============================================================================
+//
+// Up to 16 query columns per kv head.  Workgroup (h, b, z) of a grid of
+// (kv heads, sequences, S) takes the z-th of s equal shares of the pair's n
+// chunks, s = min(S, ceil(n / kSplitChunks)) from the sequence's own length
+// (the others end at once), and its waves take equal shares of those: no
+// scan over the batch and no walk, so the first loads leave after one chain
+// of kernel arguments, length and page index.
+//
+// Small calls are bound by such chains: the second kernel that the slot
+// schedules and the balanced split need takes 7 to 8 us behind the first,
+// and folding the waves' states by (column, 8 dims) per thread took up to 8k
+// cycles of a 16k-cycle decode of 512 tokens.  So here
+//  * the waves' states meet in LDS in register order and wave j folds the
+//    16-dim tile j of every state: one 16-byte read per state and lane;
+//  * the s workgroups of a pair leave their folded states in workspace slots
+//    with agent-scope stores (written through the XCD's own L2), count
+//    themselves in the pair's counter once the stores have retired, and the
+//    last one folds the slots, read with agent-scope loads.  It resets the
+//    counter, so counters that are zero before a launch are zero after it.
+//    Nothing waits for another workgroup, and there is no release fence
+//    (whose L2 write-back costs more than the second kernel).
+//
+// kSplitChunks: a further split costs a workgroup about 5k cycles (stores,
+// count, loads), a chunk per wave about 2.5k.
+#ifndef PA_FP8_SPLIT_CHUNKS
+#define PA_FP8_SPLIT_CHUNKS 16
+#endif
+constexpr int kSplitChunks = PA_FP8_SPLIT_CHUNKS;
+// A folded state in LDS or a workspace slot, in the lanes' register order:
+// [8 tiles of 16 head dims][64 lanes] x 16 B of value-unit accumulators, then
+// [64 lanes] x (base-2 maximum, sum).
+constexpr int kStateBytes = 8 * 64 * 16 + 64 * 8;
+
+__device__ __forceinline__ void state_write(LDS_AS unsigned char* s, const f32x4 (&acc)[8], float m, float L, int lane) {
+#pragma unroll
+  for (int j = 0; j < 8; ++j) *(LDS_AS f32x4*)(s + j * 1024 + lane * 16) = acc[j];
+  *(LDS_AS f32x2*)(s + 8192 + lane * 8) = f32x2{m, L};
+}
+
+__device__ __forceinline__ void st_agent(void* p, uint64_t v) {
+  __hip_atomic_store((uint64_t*)p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ uint64_t ld_agent(const void* p) {
+  return __hip_atomic_load((const uint64_t*)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ uint64_t pack_f32x2(float x, float y) {
+  return (uint64_t)__float_as_uint(x) | ((uint64_t)__float_as_uint(y) << 32);
+}
+
+template <bool PER_TOKEN, bool BS16, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void pa_fp8_split_kernel(
+    const pa_fp8_stream_args a, const int32_t* __restrict__ block_tables, const int32_t* __restrict__ kv_indptr,
+    const int32_t* __restrict__ context_lengths, const float* __restrict__ key_scale,
+    const float* __restrict__ value_scale, unsigned char* __restrict__ slots, int32_t* __restrict__ counters,
+    void* __restrict__ output) {
+  constexpr int W = WAVES;
+  constexpr int kStageBytes = kKBytes + kVBytes + (PER_TOKEN ? kScaleBytes : 0);
+  constexpr int kWaveBytes = 2 * kStageBytes;
+  constexpr int kLoadsPerChunk = 8 + (PER_TOKEN ? 1 : 0);
+  constexpr int kTiles = 8 / W;  // 16-dim tiles a wave folds
+  static_assert(kStateBytes <= kWaveBytes, "a wave's state fits in its ring");
+  __shared__ __attribute__((aligned(16))) unsigned char smem[W * kWaveBytes + 16];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int grp = lane >> 4;
+  const int c16 = lane & 15;
+  const int h = blockIdx.x, b = blockIdx.y, z = blockIdx.z;
+  const int S = gridDim.z;
+  const int ql = a.query_length;
+  const int gqa = a.query_group_size;
+  const int eq = ql * gqa;
+  const int bs = a.block_size;
+  const int bs_shift = BS16 ? 4 : __builtin_ctz((unsigned)bs);
+  const int nblocks = a.num_blocks;
+
+  Piece p;
+  piece_sequence(p, a, kv_indptr, context_lengths, b);
+  const int first = p.lo_all & ~(kChunk - 1);
+  const int n = p.hi_all > p.lo_all ? pa_cdiv(p.hi_all - first, kChunk) : 0;
+  // Shares: uniform over the pair's workgroups.
+  const int need = (n + kSplitChunks - 1) / kSplitChunks;
+  const int s = need < S ? (need > 1 ? need : 1) : S;
+  if (z >= s) return;
+
+  // Query rows of the lane's column, in flight beside the first chunk.
+  const int e = pa_min(c16, eq - 1);
+  const int qi = e / gqa;
+  const int g = e - qi * gqa;
+  const uint16_t* qp = (const uint16_t*)a.query + (int64_t)(p.orow + qi) * a.stride_q_tok +
+                       (int64_t)(h * gqa + g) * a.stride_q_head;
+  i32x4 qraw[1][4];
+  qraw[0][0] = *(const i32x4*)(qp + 16 * grp);
+  qraw[0][1] = *(const i32x4*)(qp + 16 * grp + 8);
+  qraw[0][2] = *(const i32x4*)(qp + 16 * (grp + 4));
+  qraw[0][3] = *(const i32x4*)(qp + 16 * (grp + 4) + 8);
+
+  const int w0 = (int)((int64_t)n * z / s), m = (int)((int64_t)n * (z + 1) / s) - w0;
+  const int mine0 = m * wave / W;
+  const int mine = m * (wave + 1) / W - mine0;
+  int itb = first + (w0 + mine0) * kChunk;  // first token of the next chunk to load
+  const int tb0 = itb;
+  int np0 = 0, np1 = 0;
+  auto fetch_pages = [&]() {
+    const int lp0 = itb >> bs_shift;
+    np0 = ld_uniform(block_tables, p.bt_off + pa_min(lp0, p.last_page));
+    np1 = BS16 ? ld_uniform(block_tables, p.bt_off + pa_min(lp0 + 1, p.last_page)) : np0;
+  };
+  LDS_AS unsigned char* ring = (LDS_AS unsigned char*)smem + wave * kWaveBytes;
+  auto clamp_page = [&](int q) -> int {
+    pa_note(q < 0 || q >= nblocks, PA_VIOLATION_PAGE);
+    q = q < 0 ? 0 : q;
+    return q < nblocks ? q : nblocks - 1;
+  };
+  auto issue = [&](int st) {
+    dma_chunk<PER_TOKEN, BS16>(a, key_scale, value_scale, ring + st * kStageBytes, h, itb, clamp_page(np0),
+                               BS16 ? clamp_page(np1) : 0, lane);
+    itb += kChunk;
+  };
+
+  const float k_tensor_scale = PER_TOKEN ? 1.0f : key_scale[0];
+  const float v_tensor_scale = PER_TOKEN ? 1.0f : value_scale[0];
+  WaveState<1> st;
+  st.reset();
+  if (mine > 0) {
+    fetch_pages();
+    issue(0);
+    if (mine > 1) fetch_pages();
+    QueryTile<1> qt;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) qraw[0][i] = c16 < eq ? qraw[0][i] : i32x4{0, 0, 0, 0};
+    prepare_query<1>(qt, qraw, a.query_dtype, a.softmax_scale * kLog2e * k_tensor_scale, p.ctx, ql, gqa,
+                     a.sliding_window, c16);
+    const int krow = (c16 >> 3) * kKHalf + (8 * ((c16 >> 2) & 1) + (c16 & 3)) * 16;
+    for (int k = 0; k < mine; ++k) {
+      if (k + 1 < mine) {
+        issue((k + 1) & 1);
+        if (k + 2 < mine) fetch_pages();
+        __builtin_amdgcn_s_waitcnt(vmcnt_only(kLoadsPerChunk));
+      } else {
+        __builtin_amdgcn_s_waitcnt(0);
+      }
+      compute_chunk<1, PER_TOKEN>(st, qt, ring + (k & 1) * kStageBytes, krow, grp, c16, tb0 + k * kChunk);
+    }
+  }
+
+  // ---------------- the waves' states: wave j folds tile j ----------------
+  const float vfin = PER_TOKEN ? st.vsmax : v_tensor_scale;
+  const float Lw = sum_over_groups(st.lsum[0]);
+  if (mine > 0) {
+    f32x4 v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = st.acc[0][j] * vfin;
+    state_write(ring, v, st.m2[0], Lw, lane);
+  }
+  __syncthreads();
+  float M = kNegInf, L = 0.0f;
+  f32x4 acc[kTiles];
+#pragma unroll
+  for (int t = 0; t < kTiles; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  {
+    // A wave without chunks (its share is empty) has written nothing.
+    const LDS_AS unsigned char* base = (const LDS_AS unsigned char*)smem;
+    f32x2 ml[W];
+    f32x4 x[W][kTiles];
+#pragma unroll
+    for (int r = 0; r < W; ++r) {
+      const bool live = m * (r + 1) / W > m * r / W;
+      ml[r] = f32x2{kNegInf, 0.0f};
+#pragma unroll
+      for (int t = 0; t < kTiles; ++t) x[r][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (live) {
+        ml[r] = *(const LDS_AS f32x2*)(base + r * kWaveBytes + 8192 + lane * 8);
+#pragma unroll
+        for (int t = 0; t < kTiles; ++t)
+          x[r][t] = *(const LDS_AS f32x4*)(base + r * kWaveBytes + (wave + t * W) * 1024 + lane * 16);
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < W; ++r) M = fmaxf(M, ml[r][0]);
+    const float Mu = M == kNegInf ? 0.0f : M;
+#pragma unroll
+    for (int r = 0; r < W; ++r) {
+      const float f = __builtin_amdgcn_exp2f(ml[r][0] - Mu);
+      L += ml[r][1] * f;
+#pragma unroll
+      for (int t = 0; t < kTiles; ++t) acc[t] += x[r][t] * f;
+    }
+  }
+  auto store = [&]() {
+    if (c16 >= eq) return;
+    const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+    const int64_t off = (int64_t)(p.orow + qi) * a.stride_out_tok + (int64_t)(h * gqa + g) * a.stride_out_head + 4 * grp;
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t) store_out4(output, a.output_dtype, off + 16 * (wave + t * W), acc[t] * inv);
+  };
+  if (s == 1) {
+    store();
+    return;
+  }
+
+  // ---------------- the pair's workgroups: the last one folds their states ----------------
+  const int64_t pair = (int64_t)b * a.num_kv_heads + h;
+  unsigned char* mine_slot = slots + (pair * S + z) * kStateBytes;
+  if (c16 < eq) {
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t) {
+      unsigned char* at = mine_slot + (wave + t * W) * 1024 + lane * 16;
+      st_agent(at, pack_f32x2(acc[t][0], acc[t][1]));
+      st_agent(at + 8, pack_f32x2(acc[t][2], acc[t][3]));
+    }
+    if (wave == 0) st_agent(mine_slot + 8192 + lane * 8, pack_f32x2(M, L));
+  }
+  // The state is out before the count says so.
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  LDS_AS int* flag = (LDS_AS int*)((LDS_AS unsigned char*)smem + W * kWaveBytes);
+  if (tid == 0) {
+    const int old = __hip_atomic_fetch_add(&counters[pair], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    *flag = old == s - 1;
+    if (old == s - 1) __hip_atomic_store(&counters[pair], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
+  if (__builtin_amdgcn_readfirstlane(*flag) == 0) return;
+  constexpr int kBatch = W == 8 ? 8 : 4;  // slots whose loads are in flight together
+  M = kNegInf;
+  L = 0.0f;
+#pragma unroll
+  for (int t = 0; t < kTiles; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const unsigned char* pair_slots = slots + pair * S * kStateBytes;
+  for (int i0 = 0; i0 < s; i0 += kBatch) {
+    uint64_t ml[kBatch], x[kBatch][kTiles][2];
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) {
+      const unsigned char* at = pair_slots + (int64_t)pa_min(i0 + i, s - 1) * kStateBytes;
+      ml[i] = ld_agent(at + 8192 + lane * 8);
+#pragma unroll
+      for (int t = 0; t < kTiles; ++t) {
+        x[i][t][0] = ld_agent(at + (wave + t * W) * 1024 + lane * 16);
+        x[i][t][1] = ld_agent(at + (wave + t * W) * 1024 + lane * 16 + 8);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) {
+      const bool in = i0 + i < s;
+      const float mi = in ? __uint_as_float((uint32_t)ml[i]) : kNegInf;
+      const float li = in ? __uint_as_float((uint32_t)(ml[i] >> 32)) : 0.0f;
+      const float Mn = fmaxf(M, mi);
+      const float Mu = Mn == kNegInf ? 0.0f : Mn;
+      const float f0 = __builtin_amdgcn_exp2f(M - Mu), f1 = __builtin_amdgcn_exp2f(mi - Mu);
+      L = L * f0 + li * f1;
+#pragma unroll
+      for (int t = 0; t < kTiles; ++t) {
+        const f32x4 y = {__uint_as_float((uint32_t)x[i][t][0]), __uint_as_float((uint32_t)(x[i][t][0] >> 32)),
+                         __uint_as_float((uint32_t)x[i][t][1]), __uint_as_float((uint32_t)(x[i][t][1] >> 32))};
+        acc[t] = acc[t] * f0 + y * f1;
+      }
+      M = Mn;
+    }
+  }
+  store();
+}
+
 // Cooperative column-split decode for 17..64 query columns per kv head
 // (two to four 16-column blocks).  A workgroup has one wave per column
 // block; all of its waves read the same 32-token chunks from one shared
@@ -3977,6 +4244,88 @@ hipError_t launch_bin(const pa_fp8_stream_args& a, hipStream_t s) {
   return hipGetLastError();
 }
 
+template <bool PT, bool BS16, int WAVES>
+hipError_t launch_split(const pa_fp8_stream_args& a, unsigned char* slots, int32_t* counters, hipStream_t s) {
+  const dim3 grid((unsigned)a.num_kv_heads, (unsigned)a.num_seqs, (unsigned)a.num_workers);
+  hipLaunchKernelGGL((pa_fp8_split_kernel<PT, BS16, WAVES>), grid, dim3(64 * WAVES), 0, s, a, a.block_tables,
+                     a.kv_indptr, a.context_lengths, a.key_scale, a.value_scale, slots, counters, a.output);
+  return hipGetLastError();
+}
+
+template <int WAVES>
+hipError_t dispatch_split(const pa_fp8_stream_args& a, unsigned char* slots, int32_t* counters, hipStream_t s) {
+  const bool pt = a.per_token_kv != 0, bs16 = a.block_size == 16;
+  if (pt) return bs16 ? launch_split<true, true, WAVES>(a, slots, counters, s)
+                      : launch_split<true, false, WAVES>(a, slots, counters, s);
+  return bs16 ? launch_split<false, true, WAVES>(a, slots, counters, s)
+              : launch_split<false, false, WAVES>(a, slots, counters, s);
+}
+
+// More pairs than CUs, one workgroup each: two 4-wave workgroups per CU
+// overlap each other's start and merge (512 pairs of 4096 tokens: 83.2 us; the
+// partition kernel 84.7); fewer: 8 waves, twice the loads in flight for a
+// pair.
+hipError_t dispatch_split_waves(const pa_fp8_stream_args& a, unsigned char* slots, int32_t* counters, hipStream_t s) {
+  const int cus = device_cu_count(s);
+  const bool narrow = a.num_workers == 1 && cus > 0 && (int64_t)a.num_seqs * a.num_kv_heads > cus;
+  return narrow ? dispatch_split<4>(a, slots, counters, s) : dispatch_split<8>(a, slots, counters, s);
+}
+
+// Whether an owner launch that stores no slot partials runs on the split
+// kernel: one 16-column block, grid and stride limits, and (windows) slots
+// that cover the window, since the split kernel reads all of it.
+bool split_takes(const pa_fp8_partition_args& a) {
+  const int64_t smax = 0x7fffffffLL;
+  auto fits = [&](int64_t x) { return x >= 0 && x <= smax; };
+  return a.query_length * a.query_group_size <= 16 && a.num_seqs <= 65535 && fits(a.stride_k_block) &&
+         fits(a.stride_v_block) && (!a.per_token_kv || fits(a.stride_ks_block)) &&
+         (a.sliding_window == 0 || a.num_partitions == 1 ||
+          a.num_partitions >= pa_cdiv(a.sliding_window + a.query_length - 1, PA_PARTITION_TOKENS) + 1);
+}
+
+// An owner launch as a split of one workgroup per pair.
+int split_owner(const pa_fp8_partition_args& a, hipStream_t s) {
+  pa_fp8_stream_args r = {};
+  r.abi_version = a.abi_version;
+  r.output = a.output;
+  r.query = a.query;
+  r.key_cache = a.key_cache;
+  r.value_cache = a.value_cache;
+  r.block_tables = a.block_tables;
+  r.kv_indptr = a.kv_indptr;
+  r.context_lengths = a.context_lengths;
+  r.key_scale = a.key_scale;
+  r.value_scale = a.value_scale;
+  r.stride_q_tok = a.stride_q_tok;
+  r.stride_q_head = a.stride_q_head;
+  r.stride_k_block = a.stride_k_block;
+  r.stride_k_head = a.stride_k_head;
+  r.stride_v_block = a.stride_v_block;
+  r.stride_v_head = a.stride_v_head;
+  r.stride_bt_seq = a.stride_bt_seq;
+  r.stride_ks_block = a.stride_ks_block;
+  r.stride_ks_head = a.stride_ks_head;
+  r.stride_out_tok = a.stride_out_tok;
+  r.stride_out_head = a.stride_out_head;
+  r.num_seqs = a.num_seqs;
+  r.num_kv_heads = a.num_kv_heads;
+  r.query_length = a.query_length;
+  r.query_group_size = a.query_group_size;
+  r.head_size = a.head_size;
+  r.block_size = a.block_size;
+  r.num_blocks = a.num_blocks;
+  r.max_blocks_per_seq = a.max_blocks_per_seq;
+  r.sliding_window = a.sliding_window;
+  r.per_token_kv = a.per_token_kv;
+  r.trans_v = a.trans_v;
+  r.query_dtype = a.query_dtype;
+  r.output_dtype = a.output_dtype;
+  r.num_workers = 1;
+  r.softmax_scale = a.softmax_scale;
+  const hipError_t err = dispatch_split_waves(r, nullptr, nullptr, s);
+  return err == hipSuccess ? PA_OK : (int)err;
+}
+
 // One launch of the balanced split: per-wave runs (<= 16 columns) or
 // cooperative workgroup runs.
 hipError_t dispatch_balanced(const pa_fp8_stream_args& a, hipStream_t s, int32_t* desc, float* po, float* pl) {
@@ -4161,6 +4510,7 @@ int pa_fp8_decode_partition(const pa_fp8_partition_args* a, void* stream) {
   if (generic) return generic_partition(*a, owner, (hipStream_t)stream);
   const int64_t grid = (int64_t)a->num_seqs * a->num_kv_heads * pa_cdiv(a->num_partitions, spw);
   if (grid == 0) return PA_OK;
+  if (fused && split_takes(*a)) return split_owner(*a, (hipStream_t)stream);
   if (grid > 0x7fffffffLL) return PA_ERR_SHAPE;
   const int ncg = (eq + 15) / 16;
   hipStream_t s = (hipStream_t)stream;
@@ -4282,6 +4632,30 @@ int pa_fp8_merge_balanced(const pa_fp8_stream_args* a, const void* workspace, in
     hipLaunchKernelGGL(pa_fp8_segment_merge_kernel<4>, grid, dim3(256), 0, (hipStream_t)stream, *a,
                        (const int32_t*)(ws + l.desc), (const uint16_t*)(ws + l.out), (const float*)(ws + l.lse));
   hipError_t err = hipGetLastError();
+  return err == hipSuccess ? PA_OK : (int)err;
+}
+
+int64_t pa_fp8_split_slot_bytes(int num_seqs, int num_kv_heads, int splits) {
+  if (num_seqs < 0 || num_kv_heads <= 0 || splits <= 0) return PA_ERR_SHAPE;
+  return splits == 1 ? 0 : (int64_t)num_seqs * num_kv_heads * splits * kStateBytes;
+}
+
+int pa_fp8_decode_split(const pa_fp8_stream_args* a, void* slots, int64_t slot_bytes, int32_t* counters,
+                        int64_t num_counters, void* stream) {
+  int rc = check_stream_args(a);
+  if (rc != PA_OK) return rc;
+  if (a->query_length * a->query_group_size > 16) return PA_ERR_GROUP;
+  if (a->num_workers > 65535 || a->num_seqs > 65535) return PA_ERR_SHAPE;
+  if (a->num_workers > 1) {
+    if (!slots || !counters) return PA_ERR_NULL_ARG;
+    if (((uintptr_t)slots & 15u) != 0 || ((uintptr_t)counters & 3u) != 0) return PA_ERR_ALIGN;
+    if (slot_bytes < pa_fp8_split_slot_bytes(a->num_seqs, a->num_kv_heads, a->num_workers) ||
+        num_counters < (int64_t)a->num_seqs * a->num_kv_heads)
+      return PA_ERR_SHAPE;
+  }
+  if (a->num_seqs == 0) return PA_OK;
+  const hipError_t err =
+      dispatch_split_waves(*a, (unsigned char*)slots, counters, (hipStream_t)stream);
   return err == hipSuccess ? PA_OK : (int)err;
 }
 

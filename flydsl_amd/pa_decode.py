@@ -6,13 +6,15 @@ Drop-in for the reference's Python API in kernels/pa_decode_fp8.py:
 defaults, tensor layouts, validation errors and route strings; the device
 work is done by the HIP kernels of ``libpa_fp8.so`` through its C ABI.
 
-Scheduling (see ``_schedule`` and ``_balanced_ok``): when the batch has
-enough (sequence, kv head) pairs and bounded contexts, one workgroup per
-pair walks all of its slots and merges them itself (one launch).  When the
-caller does not ask for the slot partials and the contexts may be long or
-ragged, every wave of the GPU takes an equal run of the batch's chunks
-(balanced stream split, a decode launch plus a merge launch).  Otherwise
-workgroups take one or a few slots each and the reduce kernel merges them.
+Scheduling (see ``_schedule``, ``_balanced_ok`` and ``_split_count``).  When
+the caller does not ask for the slot partials, up to 16 query columns per kv
+head: every (sequence, kv head) pair goes to a few workgroups, the last of
+which merges them (split decode, one launch); with enough pairs and bounded
+contexts one workgroup per pair (owner launch); batches whose longest
+sequence would set the duration are cut into equal runs of chunks over the
+whole GPU (balanced stream split, a decode launch plus a merge launch), as
+are 17 to 64 columns.  Otherwise workgroups take one or a few slots each and
+the reduce kernel merges them.
 
 ``exp_sums`` / ``max_logits`` / ``temporary_output`` are workspace, as in
 the reference (preallocated so that graph capture allocates nothing,
@@ -41,9 +43,11 @@ Routes (same dispatch order as the reference, :2883 / :3010 / :3123):
 
 from __future__ import annotations
 
+import collections
 import ctypes
 import functools
 import math
+import threading
 from typing import Optional
 
 import torch
@@ -254,7 +258,20 @@ def _generic_owner_ok(batch: int, kv_heads: int, eqgs: int, num_cu: int) -> bool
     return batch * kv_heads * -(-eqgs // 16) >= GENERIC_OWNER_MIN_WAVES_PER_CU * num_cu
 
 
-def _balanced_ok(route: str, batch: int, eqgs: int, user_partials: bool, owner: bool) -> bool:
+_SPLIT = "split"
+
+
+def _balanced_ok(route: str, batch: int, eqgs: int, user_partials: bool, owner: bool):
+    """Schedule of a call whose slot partials nobody reads: ``_SPLIT`` (the
+    split decode where the batch's sizes suit it, else the balanced split
+    where :func:`_stream_ok` says so), True (the balanced split) or False (the
+    slots and their reduce, or an owner launch)."""
+    if (not (user_partials or owner) and 0 < batch <= SPLIT_MAX_SEQS and eqgs <= STREAM_MAX_COLUMNS):
+        return _SPLIT
+    return _stream_ok(route, batch, eqgs, user_partials, owner)
+
+
+def _stream_ok(route: str, batch: int, eqgs: int, user_partials: bool, owner: bool) -> bool:
     """Balanced stream split for a call whose slot partials nobody reads:
     every wave (or, for more than 16 query columns, every cooperative
     workgroup) gets an equal run of the batch's chunks, so one long sequence
@@ -267,6 +284,88 @@ def _balanced_ok(route: str, batch: int, eqgs: int, user_partials: bool, owner: 
     return STREAM_MAX_COLUMNS < eqgs <= COOP_MAX_COLUMNS
 
 
+# Split decode: workgroups a pair is spread over.  As many as keep the launch
+# to one workgroup per CU (a part-filled second round costs a whole share),
+# up to SPLIT_MAX of them with at least SPLIT_CHUNKS chunks each at full
+# length; more, up to SPLIT_MOST workgroups in all, when a share would exceed
+# SPLIT_SHARE chunks.  Measured (us per call, page 16): 8 pairs of 512 tokens
+# 19.2 on the two-kernel schedules -> 6.8 with one workgroup per pair; of 8192
+# tokens 21.4 -> 13.0 with 8 (26.6 with 2, 13.1 with 16); 128 pairs of 8192
+# tokens 52.5 -> 45.8 with 2 (52.0 with 1, 49.7 with 4); 16 pairs of 8192 ..
+# 32768 tokens 37.2 -> 24.6 with 16 (28.9 with 8, 32.9 with 20: 320 workgroups).
+# Beyond SPLIT_SHARE the longest sequence's share sets the time of a ragged
+# batch (512 pairs of 1024 .. 16384 tokens: 213 with one) and equal runs over
+# the whole batch are the better schedule.
+SPLIT_CHUNKS = 16
+SPLIT_MAX = 32
+SPLIT_SHARE = 256
+SPLIT_MOST = 1024
+SPLIT_MAX_SEQS = 65535  # a grid dimension
+
+
+def _split_count(pairs: int, capacity_chunks: int, num_cu: int) -> int:
+    """Workgroups per (sequence, kv head) pair of a split decode over ``pairs``
+    pairs of at most ``capacity_chunks`` 32-token chunks each; 0 when the
+    split decode is not the schedule for them."""
+    s = min(SPLIT_MAX, max(1, num_cu // pairs))
+    s = max(1, min(s, _cdiv(capacity_chunks, SPLIT_CHUNKS)))
+    s = max(s, _cdiv(capacity_chunks, SPLIT_SHARE))
+    return s if s == 1 or pairs * s <= SPLIT_MOST else 0
+
+
+def _stream_layout_ok(output, key_cache, value_cache, key_scale, per_token_kv: bool) -> bool:
+    """Strides and alignment the streaming entry points take of a call that
+    the partition route takes too; other calls stay on that route."""
+    strides = [key_cache.stride(0), value_cache.stride(0)]
+    if per_token_kv:
+        strides.append(key_scale.stride(0))
+    return (output.data_ptr() % 16 == 0 and output.stride(0) % 8 == 0 and output.stride(1) % 8 == 0
+            and all(0 <= x <= 0x7FFFFFFF for x in strides))
+
+
+class _SplitWorkspace:
+    """State slots and pair counters of a split decode.  The counters are zero
+    between launches."""
+
+    def __init__(self, dev: torch.device, stream, nbytes: int, pairs: int):
+        # Allocated and cleared on the stream, so that the allocator orders
+        # the memory's next use after the launches that use it.
+        s = stream if isinstance(stream, torch.cuda.Stream) else torch.cuda.ExternalStream(stream.cuda_stream, dev)
+        with torch.cuda.stream(s):
+            self.slots = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+            self.counters = torch.zeros(pairs, dtype=torch.int32, device=dev)
+
+    def pointers(self):
+        return self.slots.data_ptr(), self.slots.numel(), self.counters.data_ptr(), self.counters.numel()
+
+
+# Workspaces of pa_decode_ps_launch by (device, stream): launches on a stream
+# run in order, so they share one.  The most recently used few are kept.
+_WORKSPACES_KEPT = 16
+_workspaces: "collections.OrderedDict[tuple, _SplitWorkspace]" = collections.OrderedDict()
+_workspaces_lock = threading.Lock()
+
+
+def _split_workspace(dev: torch.device, stream, pairs: int, nbytes: int, shared: bool):
+    """Workspace of a split decode on ``stream``: the stream's own
+    (``shared``), or one that belongs to the call -- a prepared call, whose
+    launches may be replayed from a graph beside other work, or a stream
+    torch does not own (its handle may come back as another stream's)."""
+    sid = getattr(stream, "stream_id", None)
+    if not shared or sid is None or not (sid == 0 or sid & 1):  # torch's own ids are 0 or odd
+        return _SplitWorkspace(dev, stream, nbytes, pairs)
+    key = (dev.index, sid)
+    with _workspaces_lock:
+        ws = _workspaces.get(key)
+        if ws is None or ws.slots.numel() < nbytes or ws.counters.numel() < pairs:
+            up = lambda x: 1 << (x - 1).bit_length()
+            ws = _workspaces[key] = _SplitWorkspace(dev, stream, up(nbytes), max(1024, up(pairs)))
+            while len(_workspaces) > _WORKSPACES_KEPT:
+                _workspaces.popitem(last=False)
+        _workspaces.move_to_end(key)
+    return ws
+
+
 class PreparedDecode:
     """A validated decode call whose C-ABI arguments are already marshalled.
 
@@ -277,13 +376,14 @@ class PreparedDecode:
     """
 
     def __init__(self, route: str, stream, keepalive, *, partition_args=None, reduce_args=None, stream_args=None,
-                 worklist_reduce_args=None, workspace=None):
+                 worklist_reduce_args=None, workspace=None, split_workspace=None):
         self.route = route
         self._pa = partition_args
         self._ra = reduce_args
         self._sa = stream_args
         self._wra = worklist_reduce_args
         self._ws = workspace
+        self._split = split_workspace
         self._keep = keepalive
         if stream is None:  # an empty batch: nothing to launch, no library needed
             self._stream = self._lib = None
@@ -314,6 +414,9 @@ class PreparedDecode:
         if wra is not None:
             return [("pa_fp8_decode_worklist", lambda: lib.pa_fp8_decode_worklist(ctypes.byref(sa), s)),
                     ("pa_fp8_reduce_worklist", lambda: lib.pa_fp8_reduce_worklist(ctypes.byref(wra), s))]
+        if self._split is not None:
+            sp, sn, cp, cn = self._split.pointers()
+            return [("pa_fp8_decode_split", lambda: lib.pa_fp8_decode_split(ctypes.byref(sa), sp, sn, cp, cn, s))]
         ws, n = self._ws.data_ptr(), self._ws.numel()
         return [("pa_fp8_decode_balanced", lambda: lib.pa_fp8_decode_balanced(ctypes.byref(sa), ws, n, s)),
                 ("pa_fp8_merge_balanced", lambda: lib.pa_fp8_merge_balanced(ctypes.byref(sa), ws, n, s))]
@@ -355,11 +458,10 @@ def pa_decode_ps_launch(
     key/value_scale: float, [1] tensor (per tensor) or [NB, Hkv, bs, 1]
     (per token per head).  Returns the route name.
     """
-    call = prepare_pa_decode(
+    call = _prepare(
         output, query, key_cache, value_cache, context_lengths, kv_page_indices, kv_indptr, softmax_scale,
-        key_scale, value_scale, sliding_window=sliding_window, metadata=metadata, block_tables=block_tables,
-        max_context_partition_num=max_context_partition_num, exp_sums=exp_sums, max_logits=max_logits,
-        temporary_output=temporary_output, stream=stream,
+        key_scale, value_scale, sliding_window, metadata, block_tables, max_context_partition_num, exp_sums,
+        max_logits, temporary_output, stream, shared_workspace=True,
     )
     return call.launch()
 
@@ -387,6 +489,16 @@ def prepare_pa_decode(
 ) -> PreparedDecode:
     """Validate and marshal one decode call (same arguments and errors as
     :func:`pa_decode_ps_launch`); returns a :class:`PreparedDecode`."""
+    return _prepare(
+        output, query, key_cache, value_cache, context_lengths, kv_page_indices, kv_indptr, softmax_scale,
+        key_scale, value_scale, sliding_window, metadata, block_tables, max_context_partition_num, exp_sums,
+        max_logits, temporary_output, stream, shared_workspace=False,
+    )
+
+
+def _prepare(output, query, key_cache, value_cache, context_lengths, kv_page_indices, kv_indptr, softmax_scale,
+             key_scale, value_scale, sliding_window, metadata, block_tables, max_context_partition_num, exp_sums,
+             max_logits, temporary_output, stream, shared_workspace: bool) -> PreparedDecode:
     num_query_heads = query.shape[1]
     num_kv_heads = key_cache.shape[1]
     trans_v = value_cache.dim() == 5
@@ -517,8 +629,36 @@ def prepare_pa_decode(
     if (generic and owner and P > 1 and not (is_graph_capturing and not have_partials)
             and not _generic_owner_ok(batch_size, num_kv_heads, eqgs, _cu_count(dev))):
         spw, owner = 1, False
-    if not generic and _balanced_ok(route, batch_size, eqgs, user_partials, owner):
-        route_name = "ps_small_block" if route == "small" else "ps_split_reduce"
+    route_name = {"sw": "ps_sw_partitioned", "small": "ps_small_block", "flat": "ps_split_reduce"}[route]
+    if route == "sw" and P <= 1:
+        route_name = "ps_sw_fused_partitioned"
+    balanced = False if generic else _balanced_ok(route, batch_size, eqgs, user_partials, owner)
+    splits = 0
+    # (a workspace whose counters are cleared by a launch is not made under
+    # capture)
+    if (balanced == _SPLIT and dev.type == "cuda" and not is_graph_capturing
+            and _stream_layout_ok(output, key_cache, value_cache, key_scale, per_token_kv)):
+        if route == "sw":
+            chunks = _cdiv(sliding_window + query_length, 32) + 1
+        else:
+            chunks = _cdiv(capacity if capacity is not None else int(kv_page_indices.numel()) * block_size, 32)
+        pairs = batch_size * num_kv_heads
+        splits = _split_count(pairs, max(1, chunks), _cu_count(dev))
+        if splits == 1:
+            spw, owner = P, True
+        elif splits > 1:
+            sa = _stream_args(output, query, key_cache, value_cache, context_lengths,
+                              kv_page_indices if route == "flat" else block_tables, kv_ind, softmax_scale, key_scale,
+                              value_scale, per_token_kv, trans_v, query_input_dtype, output_dtype, sliding_window)
+            sa.num_workers = splits
+            ws = _split_workspace(dev, s, pairs, _lib.split_slot_bytes(batch_size, num_kv_heads, splits),
+                                  shared_workspace)
+            keep = (output, query, key_cache, value_cache, context_lengths, block_tables, kv_page_indices, kv_indptr,
+                    key_scale, value_scale, ws)
+            return PreparedDecode(route_name, s, keep, stream_args=sa, split_workspace=ws)
+    if balanced == _SPLIT:
+        balanced = not owner and _stream_ok(route, batch_size, eqgs, user_partials, owner)
+    if balanced:
         sa = _stream_args(output, query, key_cache, value_cache, context_lengths,
                           kv_page_indices if route == "flat" else block_tables, kv_ind, softmax_scale, key_scale,
                           value_scale, per_token_kv, trans_v, query_input_dtype, output_dtype, sliding_window)
@@ -609,9 +749,6 @@ def prepare_pa_decode(
         pa.tmp_dtype = _tmp_dtype_code(temporary_output)
     keep = (output, query, key_cache, value_cache, context_lengths, block_tables, kv_page_indices, kv_indptr,
             key_scale, value_scale, exp_sums, max_logits, temporary_output)
-    route_name = {"sw": "ps_sw_partitioned", "small": "ps_small_block", "flat": "ps_split_reduce"}[route]
-    if route == "sw" and P <= 1:
-        route_name = "ps_sw_fused_partitioned"
     if owner:
         return PreparedDecode(route_name, s, keep, partition_args=pa)
 

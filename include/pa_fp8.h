@@ -263,7 +263,7 @@ typedef struct pa_fp8_stream_args {
   int32_t trans_v;
   int32_t query_dtype;
   int32_t output_dtype;
-  int32_t num_workers; /* balanced: runs (waves <= 16 columns, else workgroups); work list: bins */
+  int32_t num_workers; /* balanced: runs (waves <= 16 columns, else workgroups); split: splits; work list: bins */
   float softmax_scale;
 } pa_fp8_stream_args;
 
@@ -291,6 +291,22 @@ int64_t pa_fp8_balanced_workspace_bytes(int num_seqs, int num_kv_heads, int quer
  */
 int pa_fp8_decode_balanced_static(const pa_fp8_stream_args* args, void* hip_stream);
 int64_t pa_fp8_static_scratch_bytes(void);
+
+/*
+ * Split decode: up to 16 query columns per kv head in one launch, every
+ * (sequence, kv head) spread over at most num_workers workgroups (fewer for
+ * short sequences), the last of which merges them.  With num_workers > 1 it
+ * needs `slots` (pa_fp8_split_slot_bytes() bytes, contents irrelevant) and
+ * `counters` (one int32 per (sequence, kv head), zero before the first
+ * launch; every launch leaves them zero); launches that may run at the same
+ * time need buffers of their own.  Arguments and checks as
+ * pa_fp8_decode_balanced; PA_ERR_GROUP above 16 columns, PA_ERR_SHAPE above
+ * 65535 sequences or splits.
+ */
+int64_t pa_fp8_split_slot_bytes(int num_seqs, int num_kv_heads, int splits);
+int pa_fp8_decode_split(const pa_fp8_stream_args* args, void* slots, int64_t slot_bytes, int32_t* counters,
+                        int64_t num_counters, void* hip_stream);
+
 
 /* Runs a streaming launch keeps resident on num_cu CUs: waves for up to 16
  * query columns (4 per workgroup; two workgroups per CU when their LDS

@@ -1,0 +1,95 @@
+"""GPU parity of the split decode (pa_fp8_decode_split): every (sequence, kv
+head) over up to S workgroups, merged by the last one.  Edges of its ranges:
+contexts around a chunk, a share and a split, empty sequences, 1 to 16 query
+columns, both kernels' wave counts, windows, the flat page list."""
+
+from __future__ import annotations
+
+import ctypes
+
+import pytest
+import torch
+
+import flydsl_amd.pa_decode as pd
+from flydsl_amd import _lib, pa_decode_ps_launch
+from tests._cases import make_case, torch_oracle
+from tests.test_gpu_parity import assert_parity, to_dev
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+EDGES = [0, 1, 31, 32, 33, 511, 512, 513, 1024, 1025, 5000]
+SHAPES = {
+    "gqa1_edges": dict(batch=len(EDGES), num_query_heads=3, num_kv_heads=3, ctx=EDGES),
+    "gqa4_pt": dict(batch=4, num_query_heads=8, num_kv_heads=2, ctx=[1, 700, 2049, 8191], per_token=True),
+    "gqa5_page64": dict(batch=3, num_query_heads=10, num_kv_heads=2, block_size=64, ctx=[64, 65, 3000]),
+    "ql2_gqa8_pt": dict(batch=3, query_length=2, num_query_heads=16, num_kv_heads=2, ctx=[2, 517, 4100], per_token=True),
+    "ql3_gqa5": dict(batch=3, query_length=3, num_query_heads=5, num_kv_heads=1, ctx=[3, 96, 2600]),
+    "window": dict(batch=4, ctx=[5, 300, 1500, 6000], sliding_window=1000),
+    "pairs_beyond_cus": dict(batch=140, num_query_heads=8, num_kv_heads=2, ctx_range=(1, 1100)),
+}
+
+
+def split(case, S, out_dtype=torch.bfloat16):
+    out = torch.empty(case["query"].shape, dtype=out_dtype, device=DEV)
+    a = pd._stream_args(out, case["query"], case["key_cache"], case["value_cache"], case["context_lengths"],
+                        case["block_tables"], None, case["softmax_scale"], case["key_scale"], case["value_scale"],
+                        case["key_scale"].dim() > 1, True, "bf16", pd._get_output_dtype_code(out),
+                        case["sliding_window"])
+    a.num_workers = S
+    pairs = case["key_cache"].shape[1] * case["context_lengths"].shape[0]
+    # slots full of NaN: a merge that reads one its launch did not write shows
+    slots = torch.full((max(16, pairs * S * 8704),), 0xFF, dtype=torch.uint8, device=DEV)
+    counters = torch.zeros(pairs, dtype=torch.int32, device=DEV)
+    assert _lib.split_slot_bytes(case["context_lengths"].shape[0], case["key_cache"].shape[1], S) <= slots.numel()
+    s = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    outs = []
+    for _ in range(2):
+        _lib.check(_lib.load().pa_fp8_decode_split(ctypes.byref(a), slots.data_ptr(), slots.numel(),
+                                                   counters.data_ptr(), counters.numel(), s), "split")
+        torch.cuda.synchronize()
+        assert int(counters.abs().sum()) == 0
+        outs.append(out.clone())
+    assert torch.equal(outs[0], outs[1])
+    return outs[0]
+
+
+@pytest.mark.parametrize("S", [1, 2, 3, 8, 33])
+@pytest.mark.parametrize("name", sorted(SHAPES))
+def test_split_matches_oracle(name, S):
+    case = make_case(seed=len(name) + S, **SHAPES[name])
+    ctx = case["context_lengths"]
+    ref = torch_oracle(dict(case, context_lengths=ctx.clamp(min=1)), float_out=False)
+    for b in torch.nonzero(ctx == 0).flatten().tolist():
+        ref[b] = 0
+    assert_parity(split(to_dev(case), S, torch.float32 if S == 3 else torch.bfloat16), ref, f"{name}/S={S}")
+
+
+def test_launcher_shares_one_workspace_per_stream():
+    """Calls on a stream reuse its workspace, calls on two unordered streams
+    do not share one, and a prepared call has its own."""
+    case = to_dev(make_case(batch=2, ctx=[3000, 9000], num_query_heads=16, seed=5))
+    ref = torch_oracle({k: (v.cpu() if isinstance(v, torch.Tensor) else v) for k, v in case.items()}, float_out=False)
+    args = (case["query"], case["key_cache"], case["value_cache"], case["context_lengths"], None, None,
+            case["softmax_scale"], case["key_scale"], case["value_scale"])
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    outs = [torch.empty_like(case["query"]) for _ in range(8)]
+    torch.cuda.synchronize()
+    for i, out in enumerate(outs):
+        pa_decode_ps_launch(out, *args, block_tables=case["block_tables"], stream=streams[i % 2])
+    torch.cuda.synchronize()
+    for out in outs:
+        assert_parity(out, ref, "two streams")
+    spaces = [pd._split_workspace(case["query"].device, s, 4, 16, True) for s in streams]
+    assert spaces[0] is not spaces[1]
+    assert spaces[0] is pd._split_workspace(case["query"].device, streams[0], 4, 16, True)
+    assert pd._split_workspace(case["query"].device, streams[0], 4, 16, False) is not spaces[0]
+    assert len(pd._workspaces) <= pd._WORKSPACES_KEPT
+
+
+def test_split_counts():
+    assert pd._split_count(8, 2, 256) == 1 and pd._split_count(8, 16, 256) == 1  # short: one workgroup per pair
+    assert pd._split_count(8, 256, 256) == 16 and pd._split_count(128, 256, 256) == 2
+    assert pd._split_count(512, 128, 256) == 1 and pd._split_count(56, 824, 256) == 4
+    assert pd._split_count(32, 4096, 256) == 16  # shares of at most 256 chunks
+    assert pd._split_count(1024, 1024, 256) == 0  # many long pairs: equal runs over the batch
