@@ -51,6 +51,8 @@ EXPORTED_SYMBOLS = (
     "pa_fp8_decode_balanced_static",
     "pa_fp8_decode_split",
     "pa_fp8_split_slot_bytes",
+    "pa_fp8_decode_team",
+    "pa_fp8_team_slot_bytes",
     "pa_fp8_static_scratch_bytes",
     "pa_fp8_balanced_workspace_bytes",
     "pa_fp8_stream_workers",
@@ -397,6 +399,10 @@ def load(path: Optional[str] = None) -> ctypes.CDLL:
     lib.pa_fp8_decode_split.restype = ctypes.c_int
     lib.pa_fp8_split_slot_bytes.argtypes = [ctypes.c_int] * 3
     lib.pa_fp8_split_slot_bytes.restype = _i64
+    lib.pa_fp8_decode_team.argtypes = [ctypes.POINTER(StreamArgs), _vp, _i64, _vp, _i64, _vp]
+    lib.pa_fp8_decode_team.restype = ctypes.c_int
+    lib.pa_fp8_team_slot_bytes.argtypes = [ctypes.c_int]
+    lib.pa_fp8_team_slot_bytes.restype = _i64
     lib.pa_fp8_decode_balanced_static.argtypes = [ctypes.POINTER(StreamArgs), _vp]
     lib.pa_fp8_decode_balanced_static.restype = ctypes.c_int
     lib.pa_fp8_static_scratch_bytes.argtypes = []
@@ -495,6 +501,13 @@ def split_slot_bytes(num_seqs: int, num_kv_heads: int, splits: int) -> int:
     n = int(load().pa_fp8_split_slot_bytes(num_seqs, num_kv_heads, splits))
     if n < 0:
         check(n, "pa_fp8_split_slot_bytes")
+    return n
+
+
+def team_slot_bytes(num_workers: int) -> int:
+    n = int(load().pa_fp8_team_slot_bytes(num_workers))
+    if n < 0:
+        check(n, "pa_fp8_team_slot_bytes")
     return n
 
 

@@ -2547,6 +2547,514 @@ __global__ __launch_bounds__(64 * WAVES) void pa_fp8_split_kernel(
   store();
 }
 
+// ============================================================================
+// Team decode: workgroup runs of the balanced split, merged in one launch
+// ============================================================================
+//
+// Up to 16 query columns per kv head, for batches whose longest sequence
+// would set the time of a split decode.  The chunks of all (sequence, kv
+// head) pairs, laid end to end (sequence-major, kv head inner,
+// kTeamPieceCost of start cost before each pair), are cut into equal runs,
+// one 8-wave workgroup per run; the run's waves cut it again into equal
+// sub-runs.  A pair cut between the waves of one workgroup is merged in LDS,
+// one cut between workgroups by the workgroup that finishes it last, as in
+// the split decode (slots, counters, no fence, no wait), so the call is one
+// launch.  The per-wave balanced split keeps 5 to 16 columns' query images in
+// LDS at one workgroup per CU and needs the merge kernel; the slot schedule
+// that such batches took reads them with 8 slots per pair whatever their
+// lengths: 128 sequences of 16 .. 32768 tokens (lognormal), 64 query and 8 kv
+// heads, per-token scales, 204 us -> 126.
+//
+// The start search costs about 10k cycles (a scan over the batch and three
+// searches), nothing at these sizes.  Cuts: a pair of at most `snap` chunks
+// is never cut -- a boundary inside it moves to its nearer end.
+constexpr int kTeamWaves = 8;
+constexpr int kTeamPieceCost = 1;
+// A launch uses fewer workgroups before it gives one fewer chunks than this
+// (four per wave), but at least one per pair.
+#ifndef PA_FP8_TEAM_MIN
+#define PA_FP8_TEAM_MIN 32
+#endif
+constexpr int kTeamMinChunks = PA_FP8_TEAM_MIN;
+#ifndef PA_FP8_TEAM_SNAP
+#define PA_FP8_TEAM_SNAP 32
+#endif
+constexpr int kTeamSnap = PA_FP8_TEAM_SNAP;
+struct TeamPiece : Piece {
+  long long P;  // cost position of the pair's start
+  int nb, c0;   // the pair's chunks, the piece's first
+};
+
+struct TeamWalk {
+  int b, h, nb, c;
+  long long pos, end, P;
+  Piece seq;
+
+  __device__ __forceinline__ bool next(TeamPiece& p, const pa_fp8_stream_args& a, const int32_t* kv_indptr,
+                                       const int32_t* context_lengths) {
+    if (pos >= end) return false;
+    (Piece&)p = seq;
+    p.h = h;
+    p.tb0 = (seq.lo_all & ~(kChunk - 1)) + c * kChunk;
+    const long long rem = end - pos;
+    p.n = rem < nb - c ? (int)rem : nb - c;
+    p.target = -1;
+    p.desc_cnt = 0;
+    p.cut = (c > 0 ? 1 : 0) | (c + p.n < nb ? 2 : 0);
+    p.wstart = 0;
+    p.P = P;
+    p.nb = nb;
+    p.c0 = c;
+    c += p.n;
+    pos += p.n;
+    if (pos < end && c == nb) {
+      c = 0;
+      P += nb + kTeamPieceCost;
+      pos = P + kTeamPieceCost;
+      if (++h >= a.num_kv_heads) {
+        h = 0;
+        do {
+          if (b + 1 >= a.num_seqs) {  // inconsistent context lengths: stop
+            pos = end;
+            break;
+          }
+          ++b;
+          piece_sequence(seq, a, kv_indptr, context_lengths, b);
+          nb = seq.hi_all > seq.lo_all ? pa_cdiv(seq.hi_all - (seq.lo_all & ~(kChunk - 1)), kChunk) : 0;
+        } while (nb == 0);
+      }
+    }
+    return true;
+  }
+};
+
+template <bool PER_TOKEN, bool BS16>
+__global__ __launch_bounds__(64 * kTeamWaves) void pa_fp8_team_kernel(
+    const pa_fp8_stream_args a, const int32_t* __restrict__ block_tables, const int32_t* __restrict__ kv_indptr,
+    const int32_t* __restrict__ context_lengths, const float* __restrict__ key_scale,
+    const float* __restrict__ value_scale, unsigned char* __restrict__ slots, int32_t* __restrict__ counters,
+    void* __restrict__ output) {
+  constexpr int W = kTeamWaves;
+  constexpr int A = kTeamPieceCost;
+  constexpr int kStageBytes = kKBytes + kVBytes + (PER_TOKEN ? kScaleBytes : 0);
+  constexpr int kWaveBytes = 2 * kStageBytes;
+  constexpr int kLoadsPerChunk = 8 + (PER_TOKEN ? 1 : 0);
+  constexpr int kQLoads = 4;  // query row loads per lane
+  // A wave's two merge states: its ring, widened by what they need more.
+  constexpr int kWaveLds = 2 * kStateBytes > kWaveBytes ? 2 * kStateBytes : kWaveBytes;
+  __shared__ __attribute__((aligned(16))) unsigned char smem[W * kWaveLds + 64];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int grp = lane >> 4;
+  const int c16 = lane & 15;
+  const int ql = a.query_length;
+  const int gqa = a.query_group_size;
+  const int eq = ql * gqa;
+  const int bs = a.block_size;
+  const int bs_shift = BS16 ? 4 : __builtin_ctz((unsigned)bs);
+  const int nblocks = a.num_blocks;
+  const int H = a.num_kv_heads;
+  const int B = a.num_seqs;
+  const int run = blockIdx.x;
+
+  // ---------------- the run: every length loaded once and scanned ----------------
+  const int K = pa_cdiv(B, 64);  // lane l holds sequences l*K .. l*K+K-1 (K <= 16)
+  int cnt[16], rl[16];
+#pragma unroll
+  for (int k = 0; k < 16; ++k) {
+    const int bb = pa_min(lane * K + k, B - 1);
+    cnt[k] = context_lengths[bb];
+    const int32_t* rows = kv_indptr ? kv_indptr : context_lengths;
+    const int r0 = rows[bb], r1 = rows[kv_indptr ? bb + 1 : bb];
+    rl[k] = kv_indptr ? r1 - r0 : 1;
+  }
+  int mine = 0, empties = 0, live = 0;
+#pragma unroll
+  for (int k = 0; k < 16; ++k) {
+    const bool real = k < K && lane * K + k < B;
+    cnt[k] = real && rl[k] > 0 ? pa_plan_seq_chunks(cnt[k], ql, a.sliding_window) : 0;
+    mine += cnt[k] > 0 ? cnt[k] + A : 0;
+    live += cnt[k] > 0 ? 1 : 0;
+    empties |= real && cnt[k] == 0 ? 1 << k : 0;
+  }
+  // Sequences with no visible key: zero rows, one workgroup each.
+  if (wave == 0 && __ballot(empties != 0) != 0) {
+    for (int k = 0; k < K; ++k) {
+      uint64_t m = __ballot((empties >> k & 1) != 0 && (lane * K + k) % (int)gridDim.x == run);
+      while (m) {
+        const int b = (int)__builtin_ctzll(m) * K + k;
+        m &= m - 1;
+        for (int i = lane; i < ql * gqa * H * (kHead / 4); i += 64) {
+          const int d0 = 4 * (i % (kHead / 4)), qh = i / (kHead / 4) % (gqa * H), qi = i / (kHead / 4) / (gqa * H);
+          store_out4(output, a.output_dtype,
+                     (int64_t)(b * ql + qi) * a.stride_out_tok + (int64_t)qh * a.stride_out_head + d0,
+                     f32x4{0.f, 0.f, 0.f, 0.f});
+        }
+      }
+    }
+  }
+  int incl = mine;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int t = __shfl_up(incl, o, 64), u = __shfl_up(live, o, 64);
+    if (lane >= o) {
+      incl += t;
+      live += u;
+    }
+  }
+  const int excl = incl - mine;
+  const long long T = (long long)__builtin_amdgcn_readlane(incl, 63) * H;
+  if (T == 0) return;
+  const long long pairs = (long long)__builtin_amdgcn_readlane(live, 63) * H;
+  long long nwl = T / kTeamMinChunks;
+  nwl = nwl < pairs ? pairs : nwl;
+  const int nw = nwl < (long long)gridDim.x ? (int)nwl : (int)gridDim.x;
+  if (run >= nw) return;
+  const long long eighth = T / nw / 8;
+  const int snap = nw < (int)gridDim.x || eighth > kTeamSnap ? kTeamSnap : (int)eighth;
+
+  // Sequence holding cost position g (0 <= g < T): index, chunks, cost
+  // before its pairs.  Wave-uniform.
+  auto locate = [&](long long g, int& b0, int& n0, long long& base) {
+    const uint64_t hit = __ballot(mine > 0 && (long long)excl * H <= g && g < (long long)incl * H);
+    const int ls = __builtin_amdgcn_readfirstlane(hit ? (int)__builtin_ctzll(hit) : 0);
+    long long S = __builtin_amdgcn_readlane(excl, ls);
+    b0 = -1;
+    n0 = 0;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+      const int ck = __builtin_amdgcn_readlane(cnt[k], ls);
+      const int qk = ck > 0 ? ck + A : 0;
+      if (b0 < 0 && k < K) {
+        if ((S + qk) * H > g) {
+          b0 = ls * K + k;
+          n0 = ck;
+        } else {
+          S += qk;
+        }
+      }
+    }
+    base = S * H;
+  };
+  // Start of run r: an equal share of the cost, moved out of short pairs.
+  auto boundary = [&](int r) -> long long {
+    if (r <= 0) return 0;
+    if (r >= nw) return T;
+    const long long g = pa_plan_run_begin(r, T, nw);
+    int b0, n0;
+    long long base;
+    locate(g, b0, n0, base);
+    if (n0 > snap) return g;
+    const int q0 = n0 + A;
+    const int off = (int)(g - base);
+    const int o = off % q0;
+    return g - o + (2 * o >= q0 ? q0 : 0);
+  };
+  const long long g0 = boundary(run), g1 = boundary(run + 1);
+  if (g1 <= g0) return;
+  auto sub = [&](int w) -> long long { return g0 + (g1 - g0) * w / W; };
+  const long long x0 = sub(wave), x1 = sub(wave + 1);
+  TeamWalk walk;
+  walk.pos = walk.end = 0;
+  if (x1 > x0) {
+    int n0;
+    long long base;
+    locate(x0, walk.b, n0, base);
+    if (walk.b >= 0 && n0 > 0) {
+      const int off = (int)(x0 - base), q0 = n0 + A;
+      const int hh = off / q0, o = off - hh * q0;
+      walk.h = hh;
+      walk.nb = n0;
+      walk.c = o > A ? o - A : 0;  // a start inside the pair's overhead takes chunk 0
+      walk.P = base + (long long)hh * q0;
+      walk.pos = walk.P + A + walk.c;
+      walk.end = x1;
+      piece_sequence(walk.seq, a, kv_indptr, context_lengths, walk.b);
+    }
+  }
+  auto next_piece = [&](TeamPiece& p) -> bool { return walk.next(p, a, kv_indptr, context_lengths); };
+
+  LDS_AS unsigned char* ring = (LDS_AS unsigned char*)smem + wave * kWaveLds;
+  auto clamp_page = [&](int p) -> int {
+    pa_note(p < 0 || p >= nblocks, PA_VIOLATION_PAGE);
+    p = p < 0 ? 0 : p;
+    return p < nblocks ? p : nblocks - 1;
+  };
+
+  // ---------------- piece window and issue cursor (as the bin kernel) ----------------
+  TeamPiece cur, nxt;
+  bool has_cur = next_piece(cur);
+  bool has_nxt = has_cur && next_piece(nxt);
+  int itb = 0, ih = 0, ilast = 0, irem = 0, iw = 0, iorow = 0;
+  int64_t ibt = 0;
+  bool iok = false, ifirst = false;
+  int np0 = 0, np1 = 0;
+  auto fetch_pages = [&]() {
+    const int lp0 = itb >> bs_shift;
+    np0 = ld_uniform(block_tables, ibt + pa_min(lp0, ilast));
+    np1 = BS16 ? ld_uniform(block_tables, ibt + pa_min(lp0 + 1, ilast)) : np0;
+  };
+  auto issue_enter = [&](const Piece& p, int which) {
+    itb = p.tb0;
+    ih = p.h;
+    ibt = p.bt_off;
+    ilast = p.last_page;
+    irem = p.n;
+    iorow = p.orow;
+    iw = which;
+    iok = true;
+    ifirst = true;
+    fetch_pages();
+  };
+  if (has_cur) issue_enter(cur, 0);
+
+  // Query rows of the next piece, loaded into registers just before the
+  // piece's first chunk, so they retire before it.
+  i32x4 qn[4];
+  auto issue_chunk = [&](int st) -> bool {
+    const bool q = ifirst;
+    if (ifirst) {
+      const int e = pa_min(c16, eq - 1);
+      const int qi = e / gqa;
+      const int g = e - qi * gqa;
+      const uint16_t* qp = (const uint16_t*)a.query + (int64_t)(iorow + qi) * a.stride_q_tok +
+                           (int64_t)(ih * gqa + g) * a.stride_q_head;
+      qn[0] = *(const i32x4*)(qp + 16 * grp);
+      qn[1] = *(const i32x4*)(qp + 16 * grp + 8);
+      qn[2] = *(const i32x4*)(qp + 16 * (grp + 4));
+      qn[3] = *(const i32x4*)(qp + 16 * (grp + 4) + 8);
+      ifirst = false;
+    }
+    dma_chunk<PER_TOKEN, BS16>(a, key_scale, value_scale, ring + st * kStageBytes, ih, itb, clamp_page(np0),
+                               BS16 ? clamp_page(np1) : 0, lane);
+    itb += kChunk;
+    if (--irem > 0)
+      fetch_pages();
+    else if (iw == 0 && has_nxt)
+      issue_enter(nxt, 1);
+    else
+      iok = false;
+    return q;
+  };
+
+  // ---------------- compute side ----------------
+  const float k_tensor_scale = PER_TOKEN ? 1.0f : key_scale[0];
+  const float v_tensor_scale = PER_TOKEN ? 1.0f : value_scale[0];
+  const float logit_scale = a.softmax_scale * kLog2e * k_tensor_scale;
+  const int krow = (c16 >> 3) * kKHalf + (8 * ((c16 >> 2) & 1) + (c16 & 3)) * 16;
+  WaveState<1> st;
+  st.reset();
+  QueryTile<1> qt;
+  // The wave's first piece, when cut: its state waits in registers until the
+  // ring is free (value units).
+  f32x4 accA[8];
+  float mA = kNegInf, LA = 0.0f;
+  bool hasA = false, hasB = false;
+  TeamPiece pA, pB;
+  bool first_piece = true;
+  int gc = 0;
+  if (iok) issue_chunk(0);
+  int issued = 1;
+  while (has_cur) {
+    for (int k = 0; k < cur.n; ++k) {
+      const int stg = gc & 1;
+      if (issued == gc) {
+        issue_chunk(stg);
+        ++issued;
+      }
+      if (k == 0) {
+        // [query rows][chunk gc] are the newest loads: wait for the rows
+        // and turn them into operands before the next issue reuses qn.
+        __builtin_amdgcn_s_waitcnt(vmcnt_only(kLoadsPerChunk));
+        i32x4 qraw[1][4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) qraw[0][i] = c16 < eq ? qn[i] : i32x4{0, 0, 0, 0};
+        prepare_query<1>(qt, qraw, a.query_dtype, logit_scale, cur.ctx, ql, gqa, a.sliding_window, c16);
+      }
+      if (iok) {
+        ++issued;
+        if (issue_chunk(stg ^ 1))
+          __builtin_amdgcn_s_waitcnt(vmcnt_only(kLoadsPerChunk + kQLoads));
+        else
+          __builtin_amdgcn_s_waitcnt(vmcnt_only(kLoadsPerChunk));
+      } else {
+        __builtin_amdgcn_s_waitcnt(0);
+      }
+      ++gc;
+      compute_chunk<1, PER_TOKEN>(st, qt, ring + stg * kStageBytes, krow, grp, c16, cur.tb0 + k * kChunk);
+    }
+    // ---- the piece is complete ----
+    const float vfin = PER_TOKEN ? st.vsmax : v_tensor_scale;
+    const float L = sum_over_groups(st.lsum[0]);
+    if (cur.cut == 0) {
+      store_piece<true>(a, output, nullptr, nullptr, cur, st.acc[0], L, st.m2[0], vfin, c16, grp);
+    } else if (first_piece) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) accA[j] = st.acc[0][j] * vfin;
+      mA = st.m2[0];
+      LA = L;
+      pA = cur;
+      hasA = true;
+    } else {
+      // A cut piece that is not the wave's first ends its run: nothing is
+      // in flight any more, so its state goes to the ring's second slot.
+      f32x4 acc[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) acc[j] = st.acc[0][j] * vfin;
+      state_write(ring + kStateBytes, acc, st.m2[0], L, lane);
+      pB = cur;
+      hasB = true;
+    }
+    first_piece = false;
+    st.reset();
+    cur = nxt;
+    has_cur = has_nxt;
+    has_nxt = has_cur && next_piece(nxt);
+    if (iw == 1) iw = 0;
+    if (!iok && has_nxt) issue_enter(nxt, 1);
+  }
+
+  // ---------------- cut pairs: merge across the waves ----------------
+  // Every load of this wave has retired (its last chunk waited for all).
+  if (hasA) state_write(ring, accA, mA, LA, lane);
+  // Per workgroup-cut pair this workgroup finished last (first and last pair
+  // of the run): pieces, first run, sequence, kv head.
+  LDS_AS int* flags = (LDS_AS int*)((LDS_AS unsigned char*)smem + W * kWaveLds);
+  if (tid < 8) flags[tid] = 0;
+  __syncthreads();
+  // The wave holding a pair's last chunk of this run folds the pair's pieces:
+  // wave r's sits in r's first slot when r's sub-run starts inside the pair,
+  // else in r's second slot.
+#pragma unroll
+  for (int which = 0; which < 2; ++which) {
+    if (!(which == 0 ? hasA : hasB)) continue;
+    const TeamPiece p = which == 0 ? pA : pB;
+    const long long q0 = p.P + A;  // position of the pair's chunk 0
+    const int cs = g0 > q0 ? (int)(g0 - q0) : 0;
+    const int ce = g1 < q0 + p.nb ? (int)(g1 - q0) : p.nb;
+    if (p.c0 + p.n != ce) continue;  // a later wave holds the end
+    auto slot_of = [&](int r) -> int {
+      const long long xr = sub(r), xn = sub(r + 1);
+      const long long lo = xr > q0 ? xr : q0;
+      const long long hi = xn < q0 + p.nb ? xn : q0 + p.nb;
+      return lo >= hi ? -1 : r * kWaveLds + (xr >= p.P ? 0 : kStateBytes);
+    };
+    float M = kNegInf;
+    for (int r = 0; r <= wave; ++r) {
+      const int at = slot_of(r);
+      if (at >= 0) M = fmaxf(M, (*(const LDS_AS f32x2*)((LDS_AS unsigned char*)smem + at + 8192 + lane * 8))[0]);
+    }
+    const float Mu = M == kNegInf ? 0.0f : M;
+    float L = 0.0f;
+    f32x4 acc[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int r = 0; r <= wave; ++r) {
+      const int at = slot_of(r);
+      if (at < 0) continue;
+      const LDS_AS unsigned char* f = (const LDS_AS unsigned char*)smem + at;
+      const f32x2 ml = *(const LDS_AS f32x2*)(f + 8192 + lane * 8);
+      const float fr = __builtin_amdgcn_exp2f(ml[0] - Mu);
+      L += ml[1] * fr;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) acc[j] += *(const LDS_AS f32x4*)(f + j * 1024 + lane * 16) * fr;
+    }
+    if (cs == 0 && ce == p.nb) {
+      store_piece<true>(a, output, nullptr, nullptr, p, acc, L, M, 1.0f, c16, grp);
+      continue;
+    }
+    // Cut between workgroups: the state goes to the run's slot for pairs
+    // that began before it (0) or in it (1).
+    const int side = cs > 0 ? 0 : 1;
+    unsigned char* s = slots + (int64_t)(2 * run + side) * kStateBytes;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      st_agent(s + j * 1024 + lane * 16, pack_f32x2(acc[j][0], acc[j][1]));
+      st_agent(s + j * 1024 + lane * 16 + 8, pack_f32x2(acc[j][2], acc[j][3]));
+    }
+    st_agent(s + 8192 + lane * 8, pack_f32x2(M, L));
+    const int rf = pa_plan_run_of_chunk(q0, T, nw);
+    const int pieces = pa_plan_run_of_chunk(q0 + p.nb - 1, T, nw) - rf + 1;
+    // The state is out before the count says so.
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (lane == 0) {
+      const int old = __hip_atomic_fetch_add(&counters[(int64_t)p.b * H + p.h], 1, __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_AGENT);
+      if (old == pieces - 1) {
+        flags[4 * side] = pieces;
+        flags[4 * side + 1] = rf;
+        flags[4 * side + 2] = p.b;
+        flags[4 * side + 3] = p.h;
+      }
+    }
+  }
+  __syncthreads();
+  // ---------------- pairs this workgroup finished: merge their runs ----------------
+  for (int side = 0; side < 2; ++side) {
+    const int pieces = __builtin_amdgcn_readfirstlane(flags[4 * side]);
+    if (pieces == 0) continue;
+    const int rf = __builtin_amdgcn_readfirstlane(flags[4 * side + 1]);
+    Piece p;
+    p.b = __builtin_amdgcn_readfirstlane(flags[4 * side + 2]);
+    p.h = __builtin_amdgcn_readfirstlane(flags[4 * side + 3]);
+    p.orow = p.b * ql;
+    p.target = -1;
+    // Wave w folds pieces w, w + W, ...: slot 1 of the first run, slot 0 of
+    // every later one.
+    float M = kNegInf, L = 0.0f;
+    f32x4 acc[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int i = wave; i < pieces; i += W) {
+      const unsigned char* s = slots + (int64_t)(2 * (rf + i) + (i == 0 ? 1 : 0)) * kStateBytes;
+      uint64_t x[8][2];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        x[j][0] = ld_agent(s + j * 1024 + lane * 16);
+        x[j][1] = ld_agent(s + j * 1024 + lane * 16 + 8);
+      }
+      const uint64_t ml = ld_agent(s + 8192 + lane * 8);
+      const float m = __uint_as_float((uint32_t)ml), l = __uint_as_float((uint32_t)(ml >> 32));
+      const float Mn = fmaxf(M, m);
+      const float Mu = Mn == kNegInf ? 0.0f : Mn;
+      const float f0 = __builtin_amdgcn_exp2f(M - Mu), f1 = __builtin_amdgcn_exp2f(m - Mu);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const f32x4 y = {__uint_as_float((uint32_t)x[j][0]), __uint_as_float((uint32_t)(x[j][0] >> 32)),
+                         __uint_as_float((uint32_t)x[j][1]), __uint_as_float((uint32_t)(x[j][1] >> 32))};
+        acc[j] = acc[j] * f0 + y * f1;
+      }
+      L = L * f0 + l * f1;
+      M = Mn;
+    }
+    state_write(ring, acc, M, L, lane);
+    __syncthreads();
+    if (wave == 0) {
+      const int n = pa_min(pieces, W);
+      float Mc = kNegInf, Lc = 0.0f;
+      const LDS_AS unsigned char* base = (const LDS_AS unsigned char*)smem;
+      for (int r = 0; r < n; ++r) Mc = fmaxf(Mc, (*(const LDS_AS f32x2*)(base + r * kWaveLds + 8192 + lane * 8))[0]);
+      const float Mu = Mc == kNegInf ? 0.0f : Mc;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int r = 0; r < n; ++r) {
+        const LDS_AS unsigned char* f = base + r * kWaveLds;
+        const f32x2 ml = *(const LDS_AS f32x2*)(f + 8192 + lane * 8);
+        const float fr = __builtin_amdgcn_exp2f(ml[0] - Mu);
+        Lc += ml[1] * fr;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) acc[j] += *(const LDS_AS f32x4*)(f + j * 1024 + lane * 16) * fr;
+      }
+      store_piece<true>(a, output, nullptr, nullptr, p, acc, Lc, Mc, 1.0f, c16, grp);
+      if (lane == 0)
+        __hip_atomic_store(&counters[(int64_t)p.b * H + p.h], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+  }
+}
+
 // Cooperative column-split decode for 17..64 query columns per kv head
 // (two to four 16-column blocks).  A workgroup has one wave per column
 // block; all of its waves read the same 32-token chunks from one shared
@@ -4261,6 +4769,14 @@ hipError_t dispatch_split(const pa_fp8_stream_args& a, unsigned char* slots, int
               : launch_split<false, false, WAVES>(a, slots, counters, s);
 }
 
+template <bool PT, bool BS16>
+hipError_t launch_team(const pa_fp8_stream_args& a, unsigned char* slots, int32_t* counters, hipStream_t s) {
+  hipLaunchKernelGGL((pa_fp8_team_kernel<PT, BS16>), dim3((unsigned)a.num_workers), dim3(64 * kTeamWaves), 0, s, a,
+                     a.block_tables, a.kv_indptr, a.context_lengths, a.key_scale, a.value_scale, slots, counters,
+                     a.output);
+  return hipGetLastError();
+}
+
 // More pairs than CUs, one workgroup each: two 4-wave workgroups per CU
 // overlap each other's start and merge (512 pairs of 4096 tokens: 83.2 us; the
 // partition kernel 84.7); fewer: 8 waves, twice the loads in flight for a
@@ -4656,6 +5172,32 @@ int pa_fp8_decode_split(const pa_fp8_stream_args* a, void* slots, int64_t slot_b
   if (a->num_seqs == 0) return PA_OK;
   const hipError_t err =
       dispatch_split_waves(*a, (unsigned char*)slots, counters, (hipStream_t)stream);
+  return err == hipSuccess ? PA_OK : (int)err;
+}
+
+int64_t pa_fp8_team_slot_bytes(int num_workers) {
+  return num_workers <= 0 ? PA_ERR_SHAPE : (int64_t)2 * num_workers * kStateBytes;
+}
+
+int pa_fp8_decode_team(const pa_fp8_stream_args* a, void* slots, int64_t slot_bytes, int32_t* counters,
+                       int64_t num_counters, void* stream) {
+  int rc = check_stream_args(a);
+  if (rc != PA_OK) return rc;
+  if (a->query_length * a->query_group_size > 16) return PA_ERR_GROUP;
+  if (a->num_seqs > 1024) return PA_ERR_SHAPE;
+  if (!slots || !counters) return PA_ERR_NULL_ARG;
+  if (((uintptr_t)slots & 15u) != 0 || ((uintptr_t)counters & 3u) != 0) return PA_ERR_ALIGN;
+  if (slot_bytes < (int64_t)2 * a->num_workers * kStateBytes ||
+      num_counters < (int64_t)a->num_seqs * a->num_kv_heads)
+    return PA_ERR_SHAPE;
+  if (a->num_seqs == 0) return PA_OK;
+  const bool pt = a->per_token_kv != 0, bs16 = a->block_size == 16;
+  hipStream_t s = (hipStream_t)stream;
+  unsigned char* sl = (unsigned char*)slots;
+  const hipError_t err = pt ? (bs16 ? launch_team<true, true>(*a, sl, counters, s)
+                                    : launch_team<true, false>(*a, sl, counters, s))
+                            : (bs16 ? launch_team<false, true>(*a, sl, counters, s)
+                                    : launch_team<false, false>(*a, sl, counters, s));
   return err == hipSuccess ? PA_OK : (int)err;
 }
 

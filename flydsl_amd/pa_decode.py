@@ -12,8 +12,8 @@ head: every (sequence, kv head) pair goes to a few workgroups, the last of
 which merges them (split decode, one launch); with enough pairs and bounded
 contexts one workgroup per pair (owner launch); batches whose longest
 sequence would set the duration are cut into equal runs of chunks over the
-whole GPU (balanced stream split, a decode launch plus a merge launch), as
-are 17 to 64 columns.  Otherwise workgroups take one or a few slots each and
+whole GPU (up to 4 columns: balanced stream split, a decode launch plus a
+merge launch; 5 to 16: team decode, one launch), as are 17 to 64 columns.  Otherwise workgroups take one or a few slots each and
 the reduce kernel merges them.
 
 ``exp_sums`` / ``max_logits`` / ``temporary_output`` are workspace, as in
@@ -324,7 +324,7 @@ def _stream_layout_ok(output, key_cache, value_cache, key_scale, per_token_kv: b
 
 
 class _SplitWorkspace:
-    """State slots and pair counters of a split decode.  The counters are zero
+    """State slots and pair counters of a split or team decode.  The counters are zero
     between launches."""
 
     def __init__(self, dev: torch.device, stream, nbytes: int, pairs: int):
@@ -376,7 +376,7 @@ class PreparedDecode:
     """
 
     def __init__(self, route: str, stream, keepalive, *, partition_args=None, reduce_args=None, stream_args=None,
-                 worklist_reduce_args=None, workspace=None, split_workspace=None):
+                 worklist_reduce_args=None, workspace=None, split_workspace=None, team=False):
         self.route = route
         self._pa = partition_args
         self._ra = reduce_args
@@ -384,6 +384,7 @@ class PreparedDecode:
         self._wra = worklist_reduce_args
         self._ws = workspace
         self._split = split_workspace
+        self._team = team
         self._keep = keepalive
         if stream is None:  # an empty batch: nothing to launch, no library needed
             self._stream = self._lib = None
@@ -416,7 +417,9 @@ class PreparedDecode:
                     ("pa_fp8_reduce_worklist", lambda: lib.pa_fp8_reduce_worklist(ctypes.byref(wra), s))]
         if self._split is not None:
             sp, sn, cp, cn = self._split.pointers()
-            return [("pa_fp8_decode_split", lambda: lib.pa_fp8_decode_split(ctypes.byref(sa), sp, sn, cp, cn, s))]
+            name = "pa_fp8_decode_team" if self._team else "pa_fp8_decode_split"
+            fn = getattr(lib, name)
+            return [(name, lambda: fn(ctypes.byref(sa), sp, sn, cp, cn, s))]
         ws, n = self._ws.data_ptr(), self._ws.numel()
         return [("pa_fp8_decode_balanced", lambda: lib.pa_fp8_decode_balanced(ctypes.byref(sa), ws, n, s)),
                 ("pa_fp8_merge_balanced", lambda: lib.pa_fp8_merge_balanced(ctypes.byref(sa), ws, n, s))]
@@ -646,16 +649,18 @@ def _prepare(output, query, key_cache, value_cache, context_lengths, kv_page_ind
         splits = _split_count(pairs, max(1, chunks), _cu_count(dev))
         if splits == 1:
             spw, owner = P, True
-        elif splits > 1:
+        elif splits > 1 or (eqgs > BALANCED_MAX_COLUMNS and route != "sw" and batch_size <= BALANCED_MAX_SEQS):
+            # split decode, or (no split count: many long pairs) team runs
+            # where the per-wave balanced split does not take the columns
             sa = _stream_args(output, query, key_cache, value_cache, context_lengths,
                               kv_page_indices if route == "flat" else block_tables, kv_ind, softmax_scale, key_scale,
                               value_scale, per_token_kv, trans_v, query_input_dtype, output_dtype, sliding_window)
-            sa.num_workers = splits
-            ws = _split_workspace(dev, s, pairs, _lib.split_slot_bytes(batch_size, num_kv_heads, splits),
-                                  shared_workspace)
+            sa.num_workers = splits or _cu_count(dev)
+            ws = _split_workspace(dev, s, pairs, _lib.split_slot_bytes(batch_size, num_kv_heads, splits) if splits
+                                  else _lib.team_slot_bytes(sa.num_workers), shared_workspace)
             keep = (output, query, key_cache, value_cache, context_lengths, block_tables, kv_page_indices, kv_indptr,
                     key_scale, value_scale, ws)
-            return PreparedDecode(route_name, s, keep, stream_args=sa, split_workspace=ws)
+            return PreparedDecode(route_name, s, keep, stream_args=sa, split_workspace=ws, team=splits == 0)
     if balanced == _SPLIT:
         balanced = not owner and _stream_ok(route, batch_size, eqgs, user_partials, owner)
     if balanced:

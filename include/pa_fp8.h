@@ -263,7 +263,7 @@ typedef struct pa_fp8_stream_args {
   int32_t trans_v;
   int32_t query_dtype;
   int32_t output_dtype;
-  int32_t num_workers; /* balanced: runs (waves <= 16 columns, else workgroups); split: splits; work list: bins */
+  int32_t num_workers; /* balanced: runs (waves <= 16 columns, else workgroups); split: splits; team: workgroups; work list: bins */
   float softmax_scale;
 } pa_fp8_stream_args;
 
@@ -306,6 +306,20 @@ int64_t pa_fp8_static_scratch_bytes(void);
 int64_t pa_fp8_split_slot_bytes(int num_seqs, int num_kv_heads, int splits);
 int pa_fp8_decode_split(const pa_fp8_stream_args* args, void* slots, int64_t slot_bytes, int32_t* counters,
                         int64_t num_counters, void* hip_stream);
+
+/*
+ * Team decode: the balanced decode of up to 16 query columns per kv head
+ * (ql * gqa) in one launch of num_workers 8-wave workgroups (one per CU).
+ * Pairs cut between workgroups are merged by the workgroup that finishes
+ * them last, through `slots` (pa_fp8_team_slot_bytes(num_workers) bytes,
+ * contents irrelevant) and `counters` (one int32 per (sequence, kv head),
+ * zero before the first launch; every launch leaves them zero).  Launches
+ * that may run at the same time need buffers of their own.  Same arguments,
+ * limits and checks as pa_fp8_decode_balanced; PA_ERR_GROUP above 16 columns.
+ */
+int64_t pa_fp8_team_slot_bytes(int num_workers);
+int pa_fp8_decode_team(const pa_fp8_stream_args* args, void* slots, int64_t slot_bytes, int32_t* counters,
+                       int64_t num_counters, void* hip_stream);
 
 
 /* Runs a streaming launch keeps resident on num_cu CUs: waves for up to 16

@@ -1,5 +1,6 @@
-"""GPU parity of the split decode (pa_fp8_decode_split): every (sequence, kv
-head) over up to S workgroups, merged by the last one.  Edges of its ranges:
+"""GPU parity of the split decode (pa_fp8_decode_split: every (sequence, kv
+head) over up to S workgroups, merged by the last one) and of the team decode
+(pa_fp8_decode_team: equal runs of the batch per workgroup).  Edges of its ranges:
 contexts around a chunk, a share and a split, empty sequences, 1 to 16 query
 columns, both kernels' wave counts, windows, the flat page list."""
 
@@ -30,7 +31,7 @@ SHAPES = {
 }
 
 
-def split(case, S, out_dtype=torch.bfloat16):
+def split(case, S, out_dtype=torch.bfloat16, team=False):
     out = torch.empty(case["query"].shape, dtype=out_dtype, device=DEV)
     a = pd._stream_args(out, case["query"], case["key_cache"], case["value_cache"], case["context_lengths"],
                         case["block_tables"], None, case["softmax_scale"], case["key_scale"], case["value_scale"],
@@ -41,12 +42,16 @@ def split(case, S, out_dtype=torch.bfloat16):
     # slots full of NaN: a merge that reads one its launch did not write shows
     slots = torch.full((max(16, pairs * S * 8704),), 0xFF, dtype=torch.uint8, device=DEV)
     counters = torch.zeros(pairs, dtype=torch.int32, device=DEV)
-    assert _lib.split_slot_bytes(case["context_lengths"].shape[0], case["key_cache"].shape[1], S) <= slots.numel()
+    if team:
+        slots = torch.full((_lib.team_slot_bytes(S),), 0xFF, dtype=torch.uint8, device=DEV)
+    else:
+        assert _lib.split_slot_bytes(case["context_lengths"].shape[0], case["key_cache"].shape[1], S) <= slots.numel()
+    entry = _lib.load().pa_fp8_decode_team if team else _lib.load().pa_fp8_decode_split
     s = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
     outs = []
     for _ in range(2):
-        _lib.check(_lib.load().pa_fp8_decode_split(ctypes.byref(a), slots.data_ptr(), slots.numel(),
-                                                   counters.data_ptr(), counters.numel(), s), "split")
+        _lib.check(entry(ctypes.byref(a), slots.data_ptr(), slots.numel(), counters.data_ptr(), counters.numel(), s),
+                   "split")
         torch.cuda.synchronize()
         assert int(counters.abs().sum()) == 0
         outs.append(out.clone())
@@ -63,6 +68,18 @@ def test_split_matches_oracle(name, S):
     for b in torch.nonzero(ctx == 0).flatten().tolist():
         ref[b] = 0
     assert_parity(split(to_dev(case), S, torch.float32 if S == 3 else torch.bfloat16), ref, f"{name}/S={S}")
+
+
+@pytest.mark.parametrize("workgroups", [1, 5, 64, 256])
+@pytest.mark.parametrize("name", sorted(set(SHAPES) - {"window"}))
+def test_team_matches_oracle(name, workgroups):
+    case = make_case(seed=len(name) + workgroups, **SHAPES[name])
+    ctx = case["context_lengths"]
+    ref = torch_oracle(dict(case, context_lengths=ctx.clamp(min=1)), float_out=False)
+    for b in torch.nonzero(ctx == 0).flatten().tolist():
+        ref[b] = 0
+    assert_parity(split(to_dev(case), workgroups, torch.float16 if workgroups == 5 else torch.bfloat16, team=True), ref,
+                  f"{name}/{workgroups}")
 
 
 def test_launcher_shares_one_workspace_per_stream():
