@@ -7,6 +7,7 @@ missing library is an error: there is no fallback implementation.
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 from typing import Optional
 
@@ -441,6 +442,37 @@ def load(path: Optional[str] = None) -> ctypes.CDLL:
     return lib
 
 
+# Entry points of the native call path, in the order of its table.
+_NATIVE_ENTRIES = (
+    "pa_fp8_decode_partition", "pa_fp8_decode_reduce", "pa_fp8_decode_split", "pa_fp8_decode_team",
+    "pa_fp8_split_slot_bytes", "pa_fp8_team_slot_bytes", "pa_fp8_decode_balanced", "pa_fp8_merge_balanced",
+    "pa_fp8_balanced_workspace_bytes", "pa_fp8_decode_worklist", "pa_fp8_reduce_worklist",
+    "pa_fp8_recommended_splits", "pa_fp8_rope_cache", "pa_fp8_qk_norm_rope_quant", "pa_fp8_mla_decode",
+    "pa_fp8_mla_reduce",
+)
+_NATIVE = None
+
+
+def native():
+    """The native call path (``_native``, built with the library), bound to
+    the loaded library; None where it is not built or the library is not
+    there (the Python launchers then do the whole call, or say so)."""
+    global _NATIVE
+    if _NATIVE is None:
+        try:
+            from . import _native
+        except ImportError:
+            _NATIVE = False
+            return None
+        try:
+            lib = load()
+        except LibraryNotBuilt:
+            return None
+        _native.init(tuple(ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in _NATIVE_ENTRIES), check)
+        _NATIVE = _native
+    return _NATIVE or None
+
+
 def check(rc: int, what: str) -> None:
     if rc != 0:
         msg = load().pa_fp8_error_string(rc).decode()
@@ -481,6 +513,7 @@ def recommended_splits(num_seqs, num_kv_heads, split_kv_blocks, sliding_window, 
     )
 
 
+@functools.lru_cache(maxsize=None)
 def stream_workers(num_cu: int, query_length: int, query_group_size: int, per_token_kv: bool) -> int:
     n = int(load().pa_fp8_stream_workers(num_cu, query_length, query_group_size, int(per_token_kv)))
     if n < 0:

@@ -27,6 +27,8 @@ OUTPUT = os.path.join(HERE, "libpa_fp8.so")
 # The checked build: the same kernels, which also record every index they
 # clamp (pa_fp8_debug_violations in include/pa_fp8.h).
 CHECKED_OUTPUT = os.path.join(HERE, "libpa_fp8_checked.so")
+# The native call path of the Python launchers (host code).
+NATIVE_OUTPUT = os.path.join(HERE, "_native.so")
 ARCH = "gfx950"
 
 
@@ -126,10 +128,37 @@ def build_libraries(targets=((OUTPUT, ()), (CHECKED_OUTPUT, ("PA_FP8_CHECKED",))
     return out
 
 
+def native_cmd(output: str) -> list:
+    """g++ line of the native call path: a Python extension against torch's
+    headers (host code only)."""
+    import sysconfig
+
+    import torch
+
+    t = os.path.dirname(os.path.abspath(torch.__file__))
+    lib = os.path.join(t, "lib")
+    return ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{INCLUDE}",
+            "-isystem", os.path.join(t, "include"), "-isystem", os.path.join(t, "include/torch/csrc/api/include"),
+            "-isystem", os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include"),
+            f"-I{sysconfig.get_paths()['include']}", os.path.join(CSRC, "launch.cpp"), "-o", output,
+            f"-L{lib}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python", f"-Wl,-rpath,{lib}"]
+
+
+def build_native(output: str = NATIVE_OUTPUT) -> str:
+    """Compile the native call path; returns its path."""
+    tmp = output + ".tmp"
+    res = subprocess.run(native_cmd(tmp), capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"g++ of {os.path.basename(output)} failed ({res.returncode}):\n{res.stderr}")
+    os.replace(tmp, output)
+    return output
+
+
 def build_library(output: str = OUTPUT, verbose: bool = False) -> str:
     """The release library alone; returns its path."""
     return build_libraries(((output, ()),), verbose=verbose)[0]
 
 
 if __name__ == "__main__":
-    print("\n".join(build_libraries(verbose=True)))
+    print("\n".join(build_libraries(verbose=True) + [build_native()]))

@@ -72,6 +72,11 @@ def flydsl_mla_fwd_decode(
     ``split_output`` / ``split_lse`` for :func:`mla_reduce_v1`.
     ``precise_p`` (our extension) carries the probabilities as two fp8 terms
     in the value product instead of one (the reference's arithmetic)."""
+    native = _lib.native()
+    if native is not None and native.mla_decode(query, kv_buffer, kv_page_indices, work_indptr, work_info_set,
+                                                final_output, split_output, split_lse, softmax_scale,
+                                                bool(precise_p)):
+        return
     num_heads = query.size(1)
     q_dtype = query.dtype
     kv_dtype = kv_buffer.dtype
@@ -299,6 +304,10 @@ def mla_reduce_v1(
     """Log-sum-exp merge of the split rows into ``final_output`` (call site:
     tests/kernels/test_mla_decode.py:356-365).  Every reduce group slot is
     launched; empty ones exit, so no host synchronisation is needed."""
+    native = _lib.native()
+    if native is not None and final_lse is None and native.mla_reduce(
+            partial_output, partial_lse, reduce_indptr, reduce_final_map, reduce_partial_map, final_output):
+        return
     assert partial_output.dtype == torch.float32 and partial_lse.dtype == torch.float32
     assert final_output.dtype == torch.bfloat16 and final_output.is_contiguous()
     assert partial_output.is_contiguous() and partial_lse.is_contiguous()

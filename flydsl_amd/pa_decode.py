@@ -78,7 +78,9 @@ def _device_cu_count(index: int) -> int:
     return int(torch.cuda.get_device_properties(index).multi_processor_count)
 
 
-def _cu_count(device: Optional[torch.device] = None) -> int:
+def _cu_count(device=None) -> int:
+    if isinstance(device, int):
+        return _device_cu_count(device)
     dev = torch.device("cuda") if device is None else torch.device(device)
     idx = dev.index if dev.index is not None else torch.cuda.current_device()
     return _device_cu_count(idx)
@@ -323,6 +325,55 @@ def _stream_layout_ok(output, key_cache, value_cache, key_scale, per_token_kv: b
             and all(0 <= x <= 0x7FFFFFFF for x in strides))
 
 
+# Kinds of schedule (see _plan).
+OWNER, SLOTS, SPLIT, TEAM, BALANCED = "owner", "slots", "split", "team", "balanced"
+
+
+def _plan(route: str, batch: int, kv_heads: int, P: int, eqgs: int, head_size: int, block_size: int,
+          capacity: Optional[int],
+          tokens: int, user_partials: bool, have_partials: bool, capturing: bool, one_launch: bool, per_token: bool,
+          dev):
+    """Schedule of one call: (kind, n, P), n the slots per workgroup (OWNER,
+    SLOTS), the splits per pair (SPLIT) or the workers (TEAM, BALANCED), P the
+    slot count (``P`` = 0: the recommended one).  ``capacity`` / ``tokens``: bounds
+    of a context (None for flat page lists) and of the keys a pair reads;
+    ``one_launch``: whether the call may take a schedule that keeps a
+    workspace between launches."""
+    # head sizes other than 128 and more than 64 query columns per kv head
+    # run on the library's generic kernels: no balanced split for them
+    generic = head_size != 128 or eqgs > COOP_MAX_COLUMNS
+    if P == 0:
+        P = get_recommended_splits(batch, kv_heads, split_kv_blocks=KV_COMPUTE_BLOCK // block_size
+                                   if route == "small" else 1)
+    spw = _schedule(route, batch, kv_heads, P, eqgs, capacity, _cu_count(dev) if P > 1 else 1)
+    owner = spw >= P
+    if (generic and owner and P > 1 and not (capturing and not have_partials)
+            and not _generic_owner_ok(batch, kv_heads, eqgs, _cu_count(dev))):
+        spw, owner = 1, False
+    balanced = False if generic else _balanced_ok(route, batch, eqgs, user_partials, owner)
+    if balanced == _SPLIT:
+        if one_launch:
+            splits = _split_count(batch * kv_heads, max(1, _cdiv(tokens, 32)), _cu_count(dev))
+            if splits == 1:
+                return OWNER, P, P
+            if splits > 1:
+                return SPLIT, splits, P
+            # many long pairs: team runs where the per-wave balanced split
+            # does not take the columns
+            if eqgs > BALANCED_MAX_COLUMNS and route != "sw" and batch <= BALANCED_MAX_SEQS:
+                return TEAM, _cu_count(dev), P
+        balanced = _stream_ok(route, batch, eqgs, user_partials, owner)
+    if balanced:
+        return BALANCED, _lib.stream_workers(_cu_count(dev), 1, eqgs, per_token), P
+    return (OWNER, spw, P) if owner else (SLOTS, spw, P)
+
+
+def _route_name(route: str, P: int) -> str:
+    if route == "sw":
+        return "ps_sw_fused_partitioned" if P <= 1 else "ps_sw_partitioned"
+    return "ps_small_block" if route == "small" else "ps_split_reduce"
+
+
 class _SplitWorkspace:
     """State slots and pair counters of a split or team decode.  The counters are zero
     between launches."""
@@ -334,9 +385,11 @@ class _SplitWorkspace:
         with torch.cuda.stream(s):
             self.slots = torch.empty(nbytes, dtype=torch.uint8, device=dev)
             self.counters = torch.zeros(pairs, dtype=torch.int32, device=dev)
+        self._pointers = (self.slots.data_ptr(), nbytes, self.counters.data_ptr(), pairs)
 
     def pointers(self):
-        return self.slots.data_ptr(), self.slots.numel(), self.counters.data_ptr(), self.counters.numel()
+        """(slots, bytes, counters, count)"""
+        return self._pointers
 
 
 # Workspaces of pa_decode_ps_launch by (device, stream): launches on a stream
@@ -346,15 +399,25 @@ _workspaces: "collections.OrderedDict[tuple, _SplitWorkspace]" = collections.Ord
 _workspaces_lock = threading.Lock()
 
 
-def _split_workspace(dev: torch.device, stream, pairs: int, nbytes: int, shared: bool):
+def _native_workspace(index: int, stream_id: int, pairs: int, nbytes: int):
+    """Pointers of the workspace of the current stream ``stream_id`` of device
+    ``index``, and the workspace itself for the caller to hold."""
+    ws = _workspaces.get((index, stream_id))
+    if ws is None or ws.slots.numel() < nbytes or ws.counters.numel() < pairs:
+        ws = _split_workspace(index, torch.cuda.current_stream(index), pairs, nbytes, True)
+    return ws.pointers() + (ws,)
+
+
+def _split_workspace(index: int, stream, pairs: int, nbytes: int, shared: bool):
     """Workspace of a split decode on ``stream``: the stream's own
     (``shared``), or one that belongs to the call -- a prepared call, whose
     launches may be replayed from a graph beside other work, or a stream
     torch does not own (its handle may come back as another stream's)."""
     sid = getattr(stream, "stream_id", None)
+    dev = torch.device("cuda", index)
     if not shared or sid is None or not (sid == 0 or sid & 1):  # torch's own ids are 0 or odd
         return _SplitWorkspace(dev, stream, nbytes, pairs)
-    key = (dev.index, sid)
+    key = (index, sid)
     with _workspaces_lock:
         ws = _workspaces.get(key)
         if ws is None or ws.slots.numel() < nbytes or ws.counters.numel() < pairs:
@@ -461,6 +524,14 @@ def pa_decode_ps_launch(
     key/value_scale: float, [1] tensor (per tensor) or [NB, Hkv, bs, 1]
     (per token per head).  Returns the route name.
     """
+    native = _lib.native()
+    if native is not None and stream is None:
+        route = native.pa_decode(
+            output, query, key_cache, value_cache, context_lengths, kv_page_indices, kv_indptr, softmax_scale,
+            key_scale, value_scale, sliding_window, metadata, block_tables, max_context_partition_num, exp_sums,
+            max_logits, temporary_output, _plan, _native_workspace)
+        if route is not None:
+            return route
     call = _prepare(
         output, query, key_cache, value_cache, context_lengths, kv_page_indices, kv_indptr, softmax_scale,
         key_scale, value_scale, sliding_window, metadata, block_tables, max_context_partition_num, exp_sums,
@@ -536,9 +607,6 @@ def _prepare(output, query, key_cache, value_cache, context_lengths, kv_page_ind
             f"head_dim={head_size} is not built; this library supports head_dim in {GENERIC_HEAD_SIZES} "
             "(larger heads would not fit one wave's register file).")
     eqgs = query_length * query_group_size
-    # head sizes other than 128 and more than 64 query columns per kv head
-    # run on the library's generic kernels: no balanced split for them
-    generic = head_size != 128 or eqgs > COOP_MAX_COLUMNS
     block_size = int(key_cache.shape[-2])
     if tuple(key_cache.shape[2:]) != (head_size // 16, block_size, 16):
         raise ValueError(f"key_cache must be [NB, Hkv, {head_size // 16}, bs, 16], got {tuple(key_cache.shape)}")
@@ -596,10 +664,6 @@ def _prepare(output, query, key_cache, value_cache, context_lengths, kv_page_ind
                 f"pa_decode_ps_launch: block_size={block_size} requires `block_tables` "
                 "(per-sequence physical block index table)."
             )
-        if max_context_partition_num == 0:
-            max_context_partition_num = get_recommended_splits(
-                batch_size, num_kv_heads, split_kv_blocks=KV_COMPUTE_BLOCK // block_size
-            )
     else:
         route = "flat"
         if kv_page_indices is None or kv_indptr is None:
@@ -611,8 +675,6 @@ def _prepare(output, query, key_cache, value_cache, context_lengths, kv_page_ind
                 "CUDA graph capture requires precomputed `metadata`; "
                 "call `get_pa_metadata()` before capture and pass it via `metadata=`."
             )
-        if max_context_partition_num == 0:
-            max_context_partition_num = get_recommended_splits(batch_size, num_kv_heads, split_kv_blocks=1)
         kv_ind = kv_indptr
         if metadata is not None:
             return _prepare_worklist(
@@ -625,55 +687,35 @@ def _prepare(output, query, key_cache, value_cache, context_lengths, kv_page_ind
     P = int(max_context_partition_num)
 
     capacity = None if route == "flat" else int(block_tables.shape[1]) * block_size
-    spw = _schedule(route, batch_size, num_kv_heads, P, eqgs, capacity, _cu_count(dev) if P > 1 else 1)
-    owner = spw >= P
     user_partials = exp_sums is not None or max_logits is not None or temporary_output is not None
     have_partials = exp_sums is not None and max_logits is not None and temporary_output is not None
-    if (generic and owner and P > 1 and not (is_graph_capturing and not have_partials)
-            and not _generic_owner_ok(batch_size, num_kv_heads, eqgs, _cu_count(dev))):
-        spw, owner = 1, False
-    route_name = {"sw": "ps_sw_partitioned", "small": "ps_small_block", "flat": "ps_split_reduce"}[route]
-    if route == "sw" and P <= 1:
-        route_name = "ps_sw_fused_partitioned"
-    balanced = False if generic else _balanced_ok(route, batch_size, eqgs, user_partials, owner)
-    splits = 0
+    tokens = capacity if capacity is not None else int(kv_page_indices.numel()) * block_size
+    if route == "sw":
+        tokens = min(tokens, int(sliding_window) + query_length + 32)
     # (a workspace whose counters are cleared by a launch is not made under
     # capture)
-    if (balanced == _SPLIT and dev.type == "cuda" and not is_graph_capturing
-            and _stream_layout_ok(output, key_cache, value_cache, key_scale, per_token_kv)):
-        if route == "sw":
-            chunks = _cdiv(sliding_window + query_length, 32) + 1
-        else:
-            chunks = _cdiv(capacity if capacity is not None else int(kv_page_indices.numel()) * block_size, 32)
-        pairs = batch_size * num_kv_heads
-        splits = _split_count(pairs, max(1, chunks), _cu_count(dev))
-        if splits == 1:
-            spw, owner = P, True
-        elif splits > 1 or (eqgs > BALANCED_MAX_COLUMNS and route != "sw" and batch_size <= BALANCED_MAX_SEQS):
-            # split decode, or (no split count: many long pairs) team runs
-            # where the per-wave balanced split does not take the columns
-            sa = _stream_args(output, query, key_cache, value_cache, context_lengths,
-                              kv_page_indices if route == "flat" else block_tables, kv_ind, softmax_scale, key_scale,
-                              value_scale, per_token_kv, trans_v, query_input_dtype, output_dtype, sliding_window)
-            sa.num_workers = splits or _cu_count(dev)
-            ws = _split_workspace(dev, s, pairs, _lib.split_slot_bytes(batch_size, num_kv_heads, splits) if splits
-                                  else _lib.team_slot_bytes(sa.num_workers), shared_workspace)
-            keep = (output, query, key_cache, value_cache, context_lengths, block_tables, kv_page_indices, kv_indptr,
-                    key_scale, value_scale, ws)
-            return PreparedDecode(route_name, s, keep, stream_args=sa, split_workspace=ws, team=splits == 0)
-    if balanced == _SPLIT:
-        balanced = not owner and _stream_ok(route, batch_size, eqgs, user_partials, owner)
-    if balanced:
+    one_launch = (dev.type == "cuda" and not is_graph_capturing
+                  and _stream_layout_ok(output, key_cache, value_cache, key_scale, per_token_kv))
+    kind, spw, P = _plan(route, batch_size, num_kv_heads, P, eqgs, head_size, block_size, capacity, tokens,
+                         user_partials, have_partials, is_graph_capturing, one_launch, per_token_kv, dev)
+    route_name = _route_name(route, P)
+    owner = kind == OWNER
+    if kind in (SPLIT, TEAM, BALANCED):
         sa = _stream_args(output, query, key_cache, value_cache, context_lengths,
                           kv_page_indices if route == "flat" else block_tables, kv_ind, softmax_scale, key_scale,
                           value_scale, per_token_kv, trans_v, query_input_dtype, output_dtype, sliding_window)
-        sa.num_workers = _lib.stream_workers(_cu_count(dev), query_length, query_group_size, per_token_kv)
-        nbytes = _lib.balanced_workspace_bytes(batch_size, num_kv_heads, query_length, query_group_size,
-                                               sa.num_workers)
-        ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
         keep = (output, query, key_cache, value_cache, context_lengths, block_tables, kv_page_indices, kv_indptr,
-                key_scale, value_scale, ws)
-        return PreparedDecode(route_name, s, keep, stream_args=sa, workspace=ws)
+                key_scale, value_scale)
+        sa.num_workers = spw
+        if kind == BALANCED:
+            nbytes = _lib.balanced_workspace_bytes(batch_size, num_kv_heads, query_length, query_group_size,
+                                                   sa.num_workers)
+            ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+            return PreparedDecode(route_name, s, keep + (ws,), stream_args=sa, workspace=ws)
+        ws = _split_workspace(dev.index, s, batch_size * num_kv_heads,
+                              _lib.split_slot_bytes(batch_size, num_kv_heads, spw) if kind == SPLIT
+                              else _lib.team_slot_bytes(sa.num_workers), shared_workspace)
+        return PreparedDecode(route_name, s, keep + (ws,), stream_args=sa, split_workspace=ws, team=kind == TEAM)
     # An owner launch needs no slot partials; caller buffers stay unused
     # (validated all the same, as the slot routes validate them).
     if exp_sums is not None and max_logits is not None and temporary_output is not None:

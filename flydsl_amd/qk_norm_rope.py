@@ -150,6 +150,21 @@ def flydsl_qk_norm_rope_quant(
     """Fused RMSNorm + GPT-J RoPE + optional FP8 quant for Q and KV in one
     launch (reference :739-955).  Returns ``(q_out [T, H, D], kv_out [T, D],
     q_scale [T, H, NG] or None, kv_scale [T, NG] or None)``."""
+    native = _lib.native()
+    if (native is not None and stream is None and q_out is None and kv_out is None and q_scale is None
+            and kv_scale is None and isinstance(quant, bool)):
+        group = head_dim if quant_group_size is None else quant_group_size
+        try:  # the configuration's rules, checked once
+            compile_flydsl_qk_norm_rope_quant(
+                num_q_heads=num_q_heads, head_dim=head_dim, rope_head_dim=rope_head_dim, quant=quant,
+                group_size=group, scale_dtype=scale_dtype, q_weighted=q_weight is not None)
+        except Exception:
+            pass  # reported below, after the tensors' own checks
+        else:
+            out = native.qknr(q, kv, kv_weight, cos_cache, sin_cache, positions, num_q_heads, head_dim, rope_head_dim,
+                              q_weight, quant, group, int(scale_dtype == SCALE_DTYPE_E8M0))
+            if out is not None:
+                return out
     if q.dtype != torch.bfloat16:
         raise TypeError(f"q must be bf16, got {q.dtype}")
     if kv.dtype != torch.bfloat16:

@@ -70,6 +70,9 @@ def build_fused_rope_cache_module(
     index_dtype = torch.int32 if pos_dtype == "i32" else torch.int64
     cos_cols = head_dim // 2 if reuse_freqs_front_part else head_dim
     D = head_dim
+    config = (D, int(num_q_heads), int(num_kv_heads), int(block_size), int(bool(flash_layout)),
+              int(dtype_str == "bf16"), int(bool(apply_scale)), int(bool(reuse_freqs_front_part)),
+              int(pos_dtype == "i64"))
 
     def _check(name, t, shape, dt):
         if tuple(t.shape) != tuple(shape):
@@ -156,6 +159,11 @@ def build_fused_rope_cache_module(
 
     def launch_fused_rope_cache(Q, K, V, Positions, CosCache, SinCache, SlotMapping, KeyCache, ValueCache, Q_out, K_out,
                                 num_tokens, KScale, VScale, stream=None):
+        native = _lib.native()
+        if native is not None and stream is None and native.rope(
+                config, Q, K, V, Positions, CosCache, SinCache, SlotMapping, KeyCache, ValueCache, Q_out, K_out,
+                num_tokens, KScale, VScale):
+            return
         prepare(Q, K, V, Positions, CosCache, SinCache, SlotMapping, KeyCache, ValueCache, Q_out, K_out, num_tokens,
                 KScale, VScale, stream).launch()
 

@@ -97,10 +97,10 @@ def test_launcher_shares_one_workspace_per_stream():
     torch.cuda.synchronize()
     for out in outs:
         assert_parity(out, ref, "two streams")
-    spaces = [pd._split_workspace(case["query"].device, s, 4, 16, True) for s in streams]
+    spaces = [pd._split_workspace(0, s, 4, 16, True) for s in streams]
     assert spaces[0] is not spaces[1]
-    assert spaces[0] is pd._split_workspace(case["query"].device, streams[0], 4, 16, True)
-    assert pd._split_workspace(case["query"].device, streams[0], 4, 16, False) is not spaces[0]
+    assert spaces[0] is pd._split_workspace(0, streams[0], 4, 16, True)
+    assert pd._split_workspace(0, streams[0], 4, 16, False) is not spaces[0]
     assert len(pd._workspaces) <= pd._WORKSPACES_KEPT
 
 
