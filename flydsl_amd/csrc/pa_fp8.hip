@@ -3420,6 +3420,22 @@ __global__ __launch_bounds__(64 * NW, coop_waves_per_simd(NW, WORKLIST)) void pa
   }
 }
 
+// Indices of a reduce wave's row = (i2 n1 + i1) n0 + i0, wave-uniform.  In 32
+// bits wherever the rows fit: the compiler's 64-bit division is a routine of
+// some 150 instructions, and four of them took a third of a reduce over a small
+// batch.
+struct RowIndex {
+  int i0, i1, i2;
+};
+__device__ __forceinline__ RowIndex row_index(int64_t row, int64_t rows, int n0, int n1) {
+  if (rows <= 0x7fffffffLL) {
+    const uint32_t r = (uint32_t)__builtin_amdgcn_readfirstlane((int)row);
+    const uint32_t q = r / (uint32_t)n0, c = q / (uint32_t)n1;
+    return RowIndex{(int)(r - q * (uint32_t)n0), (int)(q - c * (uint32_t)n1), (int)c};
+  }
+  return RowIndex{(int)(row % n0), (int)((row / n0) % n1), (int)(row / ((int64_t)n0 * n1))};
+}
+
 // Log-sum-exp merge of n partial rows into 2 head dims per lane:
 // lse_at(i) and row_at(i) (element offset of the row) address item i.  All
 // loads of a batch of up to kBatch rows are issued before any is used.
@@ -3453,7 +3469,7 @@ __device__ __forceinline__ void merge_rows(int n, const float* lse, const float*
     o1 *= fold;
 #pragma unroll
     for (int i = 0; i < kBatch; ++i) {
-      const float wi = __shfl(w, i, 64);
+      const float wi = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(w), i));
       if (i < nb) {
         o0 += wi * x[i][0];
         o1 += wi * x[i][1];
@@ -3502,9 +3518,8 @@ __global__ __launch_bounds__(256) void pa_fp8_segment_merge_kernel(const pa_fp8_
   const int nblk = (eq + kCols - 1) / kCols;
   const int64_t rows = (int64_t)a.num_seqs * a.num_kv_heads * nblk;
   if (row >= rows) return;
-  const int blk = (int)(row % nblk);
-  const int h = (int)((row / nblk) % a.num_kv_heads);
-  const int b = (int)(row / ((int64_t)nblk * a.num_kv_heads));
+  const RowIndex ri = row_index(row, rows, nblk, a.num_kv_heads);
+  const int blk = ri.i0, h = ri.i1, b = ri.i2;
   // The pair's descriptor is read together with its length (it is only
   // meaningful, and only used, when the pair has visible keys).
   const int ctx = a.context_lengths[b];
@@ -3595,10 +3610,10 @@ __global__ __launch_bounds__(256) void pa_fp8_worklist_reduce_kernel(const pa_fp
   const int lane = threadIdx.x & 63;
   const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   const int Hq = a.num_query_heads, mq = a.max_query_length;
-  if (row >= (int64_t)a.num_groups * mq * Hq) return;
-  const int qh = (int)(row % Hq);
-  const int qi = (int)((row / Hq) % mq);
-  const int g = (int)(row / ((int64_t)Hq * mq));
+  const int64_t rows = (int64_t)a.num_groups * mq * Hq;
+  if (row >= rows) return;
+  const RowIndex ri = row_index(row, rows, Hq, mq);
+  const int qh = ri.i0, qi = ri.i1, g = ri.i2;
   const int p0 = a.reduce_indptr[g], p1 = a.reduce_indptr[g + 1];
   if (p1 <= p0) return;
   const int qo0 = a.reduce_final_map[2 * g], qo1 = a.reduce_final_map[2 * g + 1];
@@ -3628,10 +3643,10 @@ __global__ __launch_bounds__(256) void pa_fp8_worklist_reduce8_kernel(const pa_f
   const int64_t w = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   const int Hq = a.num_query_heads, mq = a.max_query_length;
   const int nhb = Hq / 8;
-  if (w >= (int64_t)a.num_groups * mq * nhb) return;
-  const int hb = (int)(w % nhb);
-  const int qi = (int)((w / nhb) % mq);
-  const int g = (int)(w / ((int64_t)nhb * mq));
+  const int64_t waves = (int64_t)a.num_groups * mq * nhb;
+  if (w >= waves) return;
+  const RowIndex ri = row_index(w, waves, nhb, mq);
+  const int hb = ri.i0, qi = ri.i1, g = ri.i2;
   const int p0 = a.reduce_indptr[g], p1 = a.reduce_indptr[g + 1];
   if (p1 <= p0) return;
   const int qo0 = a.reduce_final_map[2 * g], qo1 = a.reduce_final_map[2 * g + 1];
@@ -3693,15 +3708,14 @@ __global__ __launch_bounds__(256) void pa_fp8_worklist_reduce8_kernel(const pa_f
 // row -- is issued before any is used, so a row costs one memory round trip
 // per 32 slots; max and sum are then reduced across the wave.
 __global__ __launch_bounds__(256) void pa_fp8_lse_reduce_kernel(const pa_fp8_reduce_args a) {
-  constexpr int kBatch = 32;
+  constexpr int kBatch = 16;
   const int lane = threadIdx.x & 63;
   const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   const int eq = a.query_length * a.query_group_size;
   const int64_t rows = (int64_t)a.num_seqs * a.num_kv_heads * eq;
   if (row >= rows) return;
-  const int e = (int)(row % eq);
-  const int h = (int)((row / eq) % a.num_kv_heads);
-  const int b = (int)(row / ((int64_t)eq * a.num_kv_heads));
+  const RowIndex ri = row_index(row, rows, eq, a.num_kv_heads);
+  const int e = ri.i0, h = ri.i1, b = ri.i2;
   const int P = a.num_partitions;
   const int64_t sbase = (int64_t)b * a.stride_es_seq + (int64_t)h * a.stride_es_head + e;
   const int64_t tbase =
@@ -3744,7 +3758,7 @@ __global__ __launch_bounds__(256) void pa_fp8_lse_reduce_kernel(const pa_fp8_red
     o1 *= fold;
 #pragma unroll
     for (int i = 0; i < kBatch; ++i) {
-      const float wi = __shfl(w, i, 64);
+      const float wi = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(w), i));
       if (i < n) {
         o0 += wi * x0[i];
         o1 += wi * x1[i];
@@ -4365,9 +4379,8 @@ __global__ __launch_bounds__(256) void pa_fp8_generic_lse_reduce_kernel(const pa
   const int eq = a.query_length * a.query_group_size;
   const int64_t rows = (int64_t)a.num_seqs * a.num_kv_heads * eq;
   if (row >= rows) return;
-  const int e = (int)(row % eq);
-  const int h = (int)((row / eq) % a.num_kv_heads);
-  const int b = (int)(row / ((int64_t)eq * a.num_kv_heads));
+  const RowIndex ri = row_index(row, rows, eq, a.num_kv_heads);
+  const int e = ri.i0, h = ri.i1, b = ri.i2;
   const int64_t sbase = (int64_t)b * a.stride_es_seq + (int64_t)h * a.stride_es_head + e;
   const int64_t tbase = (int64_t)b * a.stride_to_seq + (int64_t)h * a.stride_to_head + (int64_t)e * a.stride_to_group + lane;
   // Slots in batches of kBatch whose loads are all in flight together,
@@ -4429,10 +4442,10 @@ __global__ __launch_bounds__(256) void pa_fp8_generic_worklist_reduce_kernel(con
   const int lane = threadIdx.x & 63;
   const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   const int Hq = a.num_query_heads, mq = a.max_query_length;
-  if (row >= (int64_t)a.num_groups * mq * Hq) return;
-  const int qh = (int)(row % Hq);
-  const int qi = (int)((row / Hq) % mq);
-  const int g = (int)(row / ((int64_t)Hq * mq));
+  const int64_t rows = (int64_t)a.num_groups * mq * Hq;
+  if (row >= rows) return;
+  const RowIndex ri = row_index(row, rows, Hq, mq);
+  const int qh = ri.i0, qi = ri.i1, g = ri.i2;
   const int p0 = a.reduce_indptr[g], p1 = a.reduce_indptr[g + 1];
   if (p1 <= p0) return;
   const int qo0 = a.reduce_final_map[2 * g], qo1 = a.reduce_final_map[2 * g + 1];
@@ -4921,6 +4934,8 @@ BalancedLayout balanced_layout(int B, int H, int eq, int nw) {
 // cannot allocate.  Each device holds its own copy for the life of the
 // process; the kernels take its device address (kept per device below),
 // never this name, which in host code is only a stand-in.
+// 16-column blocks up to which the balanced merge runs four columns per wave.
+constexpr int64_t kNarrowMergeBlocks = 512;
 constexpr int64_t kStaticScratchBytes = (int64_t)64 << 20;
 static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes];
 
@@ -5135,7 +5150,12 @@ int pa_fp8_merge_balanced(const pa_fp8_stream_args* a, const void* workspace, in
   if (workspace_bytes < l.total) return PA_ERR_SHAPE;
   // Up to 4 columns: one load per piece covers them (all lanes busy); else
   // 16 columns per wave, four loads per piece.
-  const bool narrow = eq <= 4;
+  // So few 16-column blocks that they leave the chip idle take the 4-column
+  // form too: four times the waves and 16 pieces in flight instead of two (40
+  // pairs of 24 columns in up to 26 pieces: 17.3 -> 5.7 us; C5's 4096 blocks
+  // keep the wide one).
+  const int64_t blocks16 = (int64_t)a->num_seqs * a->num_kv_heads * ((eq + 15) / 16);
+  const bool narrow = eq <= 4 || blocks16 <= kNarrowMergeBlocks;
   const int cols = narrow ? 4 : 16;
   const int64_t rows = (int64_t)a->num_seqs * a->num_kv_heads * ((eq + cols - 1) / cols);
   if (rows == 0) return PA_OK;
