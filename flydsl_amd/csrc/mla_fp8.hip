@@ -708,39 +708,74 @@ __global__ __launch_bounds__(Shape<NHT>::threads, 1) void mla_fp8_decode_kernel(
 
     if (last) {
       // ---- epilogue: normalise and store the work's rows ----
+      // A lane holds 4 value dims of each 16-dim tile of one head: stored as
+      // they are, an instruction writes 16 rows 64 bytes (bf16: 32) at a
+      // time, and the 32 of them per wave took 11k cycles, as long as a
+      // block's products.  So the tiles go through LDS (the block's stage,
+      // which every wave has read once past the barrier; 9 KiB of it per
+      // wave), 8 tiles at a time, and leave as whole rows' runs of 512 bytes
+      // (256).  Rows are padded by 16 bytes against bank conflicts.
       // One accumulator tile at a time (a scheduling barrier per tile): the
       // scaled tiles would otherwise all be formed before the stores.
       agpr_settle();
+      asm volatile("s_barrier" ::: "memory");
+      constexpr int kRow = 8 * 64 + 16;  // 8 tiles of one head, float32
+      static_assert(16 * kRow <= kStageBytes / Shape<NHT>::waves, "a wave's rows fit in its part of the stage");
+      LDS_AS unsigned char* tr = lds + st * kStageBytes + w * (kStageBytes / Shape<NHT>::waves);
+      // (lane-dependent offsets from lane_id(), so that none is hoisted into
+      // the block loop)
+      const int el = lane_id();
+      LDS_AS unsigned char* to = tr + (el & 15) * kRow + (el >> 4) * 16;
       const bool direct = cur.w.pql < 0;
+      const int64_t row0 = (int64_t)(direct ? cur.w.qo : cur.w.pql) * kHeads;
 #pragma unroll
       for (int ht = 0; ht < NHT; ++ht) {
         const float l = sum_over_groups(lsum[ht]);
         const float inv = l > 0.f ? 1.f / l : 0.f;
-        const int head = 16 * NHT * w + 16 * ht + c;
-        const int64_t prow = direct ? (int64_t)cur.w.qo * kHeads + head : (int64_t)cur.w.pql * kHeads + head;
-        // the lane's value dims 4g .. 4g+3 of each 16-dim tile: one pointer,
-        // constant offsets per tile
-        unsigned char* lrow = direct ? (unsigned char*)a.final_output + prow * (kVDim * 2) + 8 * g
-                                     : (unsigned char*)(a.split_output + prow * kVDim) + 16 * g;
+        const int head0 = 16 * NHT * w + 16 * ht;
 #pragma unroll
-        for (int db = 0; db < 16; ++db)
+        for (int pass = 0; pass < 4; ++pass) {
 #pragma unroll
-          for (int rt = 0; rt < 2; ++rt) {
-            f32x4 v = read_acc(o[db][rt][ht]) * inv;
+          for (int t = 0; t < 8; ++t) {
+            f32x4 v = read_acc(o[4 * pass + (t >> 1)][t & 1][ht]) * inv;
             // an empty range (l = 0) stores zeros whatever its page held
 #pragma unroll
             for (int i = 0; i < 4; ++i) v[i] = l > 0.f ? v[i] : 0.f;
-            const int d0 = 32 * db + 16 * rt;
-            if (direct) {
-              const uint32_t lo = f32_to_bf16_bits(v[0]) | (f32_to_bf16_bits(v[1]) << 16);
-              const uint32_t hi = f32_to_bf16_bits(v[2]) | (f32_to_bf16_bits(v[3]) << 16);
-              *(i32x2*)(lrow + 2 * d0) = i32x2{(int)lo, (int)hi};
-            } else {
-              *(f32x4*)(lrow + 4 * d0) = v;
-            }
+            *(LDS_AS f32x4*)(to + t * 64) = v;
             __builtin_amdgcn_sched_barrier(0);
           }
-        if (!direct && g == 0) a.split_lse[prow] = l > 0.f ? (m0[ht] + __builtin_amdgcn_logf(l)) * kLn2 : kNegInf;
+          if (direct) {
+            // 16 bytes of bf16: 8 dims of head 4 i + lane / 16
+            const int ln = el;
+            unsigned char* at = (unsigned char*)a.final_output + (row0 + head0 + (ln >> 4)) * (kVDim * 2) + 256 * pass +
+                                16 * (ln & 15);
+            const LDS_AS unsigned char* from = tr + (ln >> 4) * kRow + 32 * (ln & 15);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              const f32x4 x = *(const LDS_AS f32x4*)(from + 4 * i * kRow);
+              const f32x4 y = *(const LDS_AS f32x4*)(from + 4 * i * kRow + 16);
+              *(i32x4*)(at + i * (4 * kVDim * 2)) =
+                  i32x4{(int)(f32_to_bf16_bits(x[0]) | (f32_to_bf16_bits(x[1]) << 16)),
+                        (int)(f32_to_bf16_bits(x[2]) | (f32_to_bf16_bits(x[3]) << 16)),
+                        (int)(f32_to_bf16_bits(y[0]) | (f32_to_bf16_bits(y[1]) << 16)),
+                        (int)(f32_to_bf16_bits(y[2]) | (f32_to_bf16_bits(y[3]) << 16))};
+              __builtin_amdgcn_sched_barrier(0);
+            }
+          } else {
+            // 4 dims of head 2 i + lane / 32
+            const int ln = el;
+            unsigned char* at = (unsigned char*)(a.split_output + (row0 + head0 + (ln >> 5)) * kVDim) + 512 * pass +
+                                16 * (ln & 31);
+            const LDS_AS unsigned char* from = tr + (ln >> 5) * kRow + 16 * (ln & 31);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+              *(f32x4*)(at + i * (2 * kVDim * 4)) = *(const LDS_AS f32x4*)(from + 2 * i * kRow);
+              __builtin_amdgcn_sched_barrier(0);
+            }
+          }
+        }
+        if (!direct && el < 16)
+          a.split_lse[row0 + head0 + el] = l > 0.f ? (m0[ht] + __builtin_amdgcn_logf(l)) * kLn2 : kNegInf;
         lsum[ht] = 0.f;
       }
     }
@@ -759,74 +794,105 @@ __global__ __launch_bounds__(Shape<NHT>::threads, 1) void mla_fp8_decode_kernel(
   }
 }
 
-// One wave per (group, head): lane l merges value dims 8l .. 8l+7.
+// One wave per (group, head, 512 / SPLIT value dims): lane l merges 8 / SPLIT
+// of them.  SPLIT = 4 where the heads alone are too few waves for the chip
+// (4 rows x 128 heads): four times the waves, each with twice the pieces in
+// flight.
+template <int SPLIT>
 __global__ __launch_bounds__(256) void mla_fp8_reduce_kernel(const pa_mla_reduce_args a) {
+  constexpr int N = 8 / SPLIT;  // value dims per lane: two 16-byte loads or one of 8 bytes
+  constexpr int kBatch = SPLIT == 1 ? 8 : 16;
+  static_assert(SPLIT == 1 || SPLIT == 4, "8 or 2 dims per lane");
   const int gidx = blockIdx.x;
-  const int head = blockIdx.y * 4 + (threadIdx.x >> 6);
+  const int unit = blockIdx.y * 4 + (threadIdx.x >> 6);
+  const int head = unit / SPLIT, part = unit % SPLIT;
   const int lane = threadIdx.x & 63;
+  const int d0 = part * (kVDim / SPLIT) + N * lane;
   int p0 = a.reduce_indptr[gidx], p1 = a.reduce_indptr[gidx + 1];
   p0 = min(max(p0, 0), a.num_partial_map);
   p1 = min(max(p1, p0), a.num_partial_map);
   if (p0 >= p1) return;
   const int row0 = min(max(a.reduce_final_map[2 * gidx], 0), a.num_rows);
   const int row1 = min(max(a.reduce_final_map[2 * gidx + 1], row0), a.num_rows);
-  // Pieces are merged in batches of kBatch whose loads (lse and the lane's
-  // 8 value dims) are all in flight together, with an online log-sum-exp:
-  // one round trip per batch instead of two per piece.  Pieces outside the
-  // split buffers or with lse -inf (no visible key) are skipped.
-  constexpr int kBatch = 8;
+  // Lane i takes piece i's row and lse, 64 pieces at a time: two round trips
+  // for all of them.  Their value dims then depend on nothing but the rows,
+  // kBatch pieces in flight together.  Pieces outside the split buffers or
+  // with lse -inf (no visible key) have weight 0 and are skipped.
   for (int row = row0; row < row1; ++row) {
     const int r = row - row0;
     float mx = kNegInf, wsum = 0.f;
-    float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    for (int i0 = p0; i0 < p1; i0 += kBatch) {
-      int64_t prow[kBatch];
-      bool ok[kBatch];
+    float acc[N];
 #pragma unroll
-      for (int k = 0; k < kBatch; ++k) {
-        const int pr = i0 + k < p1 ? a.reduce_partial_map[i0 + k] + r : -1;
-        ok[k] = pr >= 0 && pr < a.num_partial;
-        prow[k] = (int64_t)(ok[k] ? pr : 0) * kHeads + head;
-      }
-      float l[kBatch];
-      f32x4 x0[kBatch], x1[kBatch];
+    for (int j = 0; j < N; ++j) acc[j] = 0.f;
+    for (int base = p0; base < p1; base += 64) {
+      const int pr = base + lane < p1 ? a.reduce_partial_map[base + lane] + r : -1;
+      const bool ok = pr >= 0 && pr < a.num_partial;
+      const int prow = ok ? pr : 0;
+      const float l = ok ? a.split_lse[(int64_t)prow * kHeads + head] : kNegInf;
+      float mb = l;
 #pragma unroll
-      for (int k = 0; k < kBatch; ++k) {
-        l[k] = kNegInf;
-        x0[k] = x1[k] = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (ok[k]) {  // wave-uniform
-          const f32x4* src = (const f32x4*)(a.split_output + prow[k] * kVDim + 8 * lane);
-          l[k] = a.split_lse[prow[k]];
-          x0[k] = src[0];
-          x1[k] = src[1];
+      for (int o = 32; o >= 1; o >>= 1) mb = fmaxf(mb, __shfl_xor(mb, o, 64));
+      const float mn = fmaxf(mx, mb);
+      if (mn == kNegInf) continue;
+      const float w = l == kNegInf ? 0.f : __expf(l - mn);
+      float ws = w;
+#pragma unroll
+      for (int o = 32; o >= 1; o >>= 1) ws += __shfl_xor(ws, o, 64);
+      const float fold = mx == kNegInf ? 0.f : __expf(mx - mn);
+      wsum = wsum * fold + ws;
+#pragma unroll
+      for (int j = 0; j < N; ++j) acc[j] *= fold;
+      mx = mn;
+      const int n = min(64, p1 - base);
+      for (int i0 = 0; i0 < n; i0 += kBatch) {
+        float x[kBatch][N], wk[kBatch];
+#pragma unroll
+        for (int k = 0; k < kBatch; ++k) {
+          const int i = min(i0 + k, 63);
+          wk[k] = i0 + k < n ? __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(w), i)) : 0.f;
+          const int pk = __builtin_amdgcn_readlane(prow, i);
+          if (wk[k] != 0.f) {  // wave-uniform
+            const float* src = a.split_output + ((int64_t)pk * kHeads + head) * kVDim + d0;
+            if constexpr (SPLIT == 1) {
+              const f32x4 u = *(const f32x4*)src, v = *(const f32x4*)(src + 4);
+#pragma unroll
+              for (int j = 0; j < 4; ++j) {
+                x[k][j] = u[j];
+                x[k][4 + j] = v[j];
+              }
+            } else {
+              const f32x2 u = *(const f32x2*)src;
+              x[k][0] = u[0];
+              x[k][1] = u[1];
+            }
+          } else {
+#pragma unroll
+            for (int j = 0; j < N; ++j) x[k][j] = 0.f;
+          }
         }
-      }
 #pragma unroll
-      for (int k = 0; k < kBatch; ++k) {
-        if (l[k] == kNegInf) continue;
-        const float mn = fmaxf(mx, l[k]);
-        const float fold = mx == kNegInf ? 0.f : __expf(mx - mn);
-        const float w = __expf(l[k] - mn);
+        for (int k = 0; k < kBatch; ++k)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          acc[j] = acc[j] * fold + w * x0[k][j];
-          acc[4 + j] = acc[4 + j] * fold + w * x1[k][j];
-        }
-        wsum = wsum * fold + w;
-        mx = mn;
+          for (int j = 0; j < N; ++j) acc[j] += wk[k] * x[k][j];
       }
     }
     const float inv = wsum > 0.f ? 1.f / wsum : 0.f;
-    uint32_t packed[4];
+    uint32_t packed[N / 2];
 #pragma unroll
-    for (int k = 0; k < 4; ++k)
+    for (int k = 0; k < N / 2; ++k)
       packed[k] = f32_to_bf16_bits(acc[2 * k] * inv) | (f32_to_bf16_bits(acc[2 * k + 1] * inv) << 16);
-    unsigned char* orow = (unsigned char*)a.final_output + ((int64_t)row * kHeads + head) * (kVDim * 2);
-    *(i32x4*)(orow + 16 * lane) = i32x4{(int)packed[0], (int)packed[1], (int)packed[2], (int)packed[3]};
-    if (a.final_lse && lane == 0)
+    unsigned char* orow = (unsigned char*)a.final_output + ((int64_t)row * kHeads + head) * (kVDim * 2) + 2 * d0;
+    if constexpr (SPLIT == 1)
+      *(i32x4*)orow = i32x4{(int)packed[0], (int)packed[1], (int)packed[2], (int)packed[3]};
+    else
+      *(uint32_t*)orow = packed[0];
+    if (a.final_lse && lane == 0 && part == 0)
       a.final_lse[(int64_t)row * kHeads + head] = wsum > 0.f ? mx + __logf(wsum) : kNegInf;
   }
 }
+
+// Groups (query rows) up to which the reduce splits the value dims.
+constexpr int kSplitReduceGroups = 8;
 
 bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 
@@ -947,7 +1013,10 @@ extern "C" int pa_fp8_mla_reduce(const pa_mla_reduce_args* a, void* stream) {
   if (a->num_partial > 0 && (!a->split_output || !a->split_lse || !a->reduce_partial_map)) return PA_ERR_NULL_ARG;
   if (!aligned16(a->final_output) || (a->split_output && !aligned16(a->split_output))) return PA_ERR_ALIGN;
   hipStream_t s = (hipStream_t)stream;
-  hipLaunchKernelGGL(mla_fp8_reduce_kernel, dim3(a->num_groups, kHeads / 4), dim3(256), 0, s, *a);
+  if (a->num_groups <= kSplitReduceGroups)
+    hipLaunchKernelGGL(mla_fp8_reduce_kernel<4>, dim3(a->num_groups, kHeads), dim3(256), 0, s, *a);
+  else
+    hipLaunchKernelGGL(mla_fp8_reduce_kernel<1>, dim3(a->num_groups, kHeads / 4), dim3(256), 0, s, *a);
   return (int)hipGetLastError();
 }
 
