@@ -302,16 +302,30 @@ SPLIT_CHUNKS = 16
 SPLIT_MAX = 32
 SPLIT_SHARE = 256
 SPLIT_MOST = 1024
+SPLIT_EVEN = 128
+SPLIT_FEW = 64
 SPLIT_MAX_SEQS = 65535  # a grid dimension
 
 
-def _split_count(pairs: int, capacity_chunks: int, num_cu: int) -> int:
+def _split_count(pairs: int, capacity_chunks: int, num_cu: int, bounded: bool = False) -> int:
     """Workgroups per (sequence, kv head) pair of a split decode over ``pairs``
-    pairs of at most ``capacity_chunks`` 32-token chunks each; 0 when the
-    split decode is not the schedule for them."""
+    pairs of at most ``capacity_chunks`` 32-token chunks each (``bounded``: by
+    a window, so that they hardly differ); 0 when the split decode is not the
+    schedule for them."""
     s = min(SPLIT_MAX, max(1, num_cu // pairs))
     s = max(1, min(s, _cdiv(capacity_chunks, SPLIT_CHUNKS)))
     s = max(s, _cdiv(capacity_chunks, SPLIT_SHARE))
+    if not bounded and capacity_chunks > SPLIT_EVEN:
+        # Uneven pairs, each a large part of a CU's work: in more workgroups
+        # than CUs, or one to a CU where the longest takes twice the mean,
+        # equal runs are faster (212 pairs, lognormal up to 9970 tokens: 43.0
+        # us balanced, 50.5 with 2; 200 pairs up to 8192, 16 columns: 42.2
+        # with 1, team runs 32.7).  Few pairs still gain from one launch (64
+        # pairs of 4096 .. 32768 tokens: 75.7 balanced, 69.7 with 4).
+        if s > 1 and pairs > SPLIT_FEW and pairs * s > num_cu:
+            return 0
+        if s == 1 and num_cu // 2 < pairs < 2 * num_cu:
+            return 0
     return s if s == 1 or pairs * s <= SPLIT_MOST else 0
 
 
@@ -353,7 +367,7 @@ def _plan(route: str, batch: int, kv_heads: int, P: int, eqgs: int, head_size: i
     balanced = False if generic else _balanced_ok(route, batch, eqgs, user_partials, owner)
     if balanced == _SPLIT:
         if one_launch:
-            splits = _split_count(batch * kv_heads, max(1, _cdiv(tokens, 32)), _cu_count(dev))
+            splits = _split_count(batch * kv_heads, max(1, _cdiv(tokens, 32)), _cu_count(dev), route == "sw")
             if splits == 1:
                 return OWNER, P, P
             if splits > 1:

@@ -109,4 +109,8 @@ def test_split_counts():
     assert pd._split_count(8, 256, 256) == 16 and pd._split_count(128, 256, 256) == 2
     assert pd._split_count(512, 128, 256) == 1 and pd._split_count(56, 824, 256) == 4
     assert pd._split_count(32, 4096, 256) == 16  # shares of at most 256 chunks
+    # uneven pairs that are large parts of a CU's work: equal runs, unless few
+    assert pd._split_count(212, 312, 256) == 0 and pd._split_count(200, 256, 256) == 0
+    assert pd._split_count(200, 256, 256, True) == 1 and pd._split_count(200, 128, 256) == 1
+    assert pd._split_count(64, 975, 256) == 4
     assert pd._split_count(1024, 1024, 256) == 0  # many long pairs: equal runs over the batch
