@@ -815,8 +815,9 @@ __global__ __launch_bounds__(256) void mla_fp8_reduce_kernel(const pa_mla_reduce
   const int row0 = min(max(a.reduce_final_map[2 * gidx], 0), a.num_rows);
   const int row1 = min(max(a.reduce_final_map[2 * gidx + 1], row0), a.num_rows);
   // Lane i takes piece i's row and lse, 64 pieces at a time: two round trips
-  // for all of them.  Their value dims then depend on nothing but the rows,
-  // kBatch pieces in flight together.  Pieces outside the split buffers or
+  // for all of them.  The value dims depend on nothing but the rows: the first
+  // kBatch pieces are loaded beside the lse, ahead of the weights (128 groups:
+  // 17.3 us with the loads behind the weights, 15.4 so).  Pieces outside the split buffers or
   // with lse -inf (no visible key) have weight 0 and are skipped.
   for (int row = row0; row < row1; ++row) {
     const int r = row - row0;
@@ -825,10 +826,35 @@ __global__ __launch_bounds__(256) void mla_fp8_reduce_kernel(const pa_mla_reduce
 #pragma unroll
     for (int j = 0; j < N; ++j) acc[j] = 0.f;
     for (int base = p0; base < p1; base += 64) {
+      const int n = min(64, p1 - base);
       const int pr = base + lane < p1 ? a.reduce_partial_map[base + lane] + r : -1;
       const bool ok = pr >= 0 && pr < a.num_partial;
-      const int prow = ok ? pr : 0;
-      const float l = ok ? a.split_lse[(int64_t)prow * kHeads + head] : kNegInf;
+      const int prow = ok ? pr : -1;
+      const float l = ok ? a.split_lse[(int64_t)pr * kHeads + head] : kNegInf;
+      float x[kBatch][N];
+      auto load = [&](int i0) {
+#pragma unroll
+        for (int k = 0; k < kBatch; ++k) {
+          const int pk = i0 + k < n ? __builtin_amdgcn_readlane(prow, min(i0 + k, 63)) : -1;
+#pragma unroll
+          for (int j = 0; j < N; ++j) x[k][j] = 0.f;
+          if (pk < 0) continue;  // wave-uniform
+          const float* src = a.split_output + ((int64_t)pk * kHeads + head) * kVDim + d0;
+          if constexpr (SPLIT == 1) {
+            const f32x4 u = *(const f32x4*)src, v = *(const f32x4*)(src + 4);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              x[k][j] = u[j];
+              x[k][4 + j] = v[j];
+            }
+          } else {
+            const f32x2 u = *(const f32x2*)src;
+            x[k][0] = u[0];
+            x[k][1] = u[1];
+          }
+        }
+      };
+      load(0);
       float mb = l;
 #pragma unroll
       for (int o = 32; o >= 1; o >>= 1) mb = fmaxf(mb, __shfl_xor(mb, o, 64));
@@ -843,37 +869,16 @@ __global__ __launch_bounds__(256) void mla_fp8_reduce_kernel(const pa_mla_reduce
 #pragma unroll
       for (int j = 0; j < N; ++j) acc[j] *= fold;
       mx = mn;
-      const int n = min(64, p1 - base);
       for (int i0 = 0; i0 < n; i0 += kBatch) {
-        float x[kBatch][N], wk[kBatch];
+        if (i0 > 0) load(i0);
 #pragma unroll
         for (int k = 0; k < kBatch; ++k) {
-          const int i = min(i0 + k, 63);
-          wk[k] = i0 + k < n ? __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(w), i)) : 0.f;
-          const int pk = __builtin_amdgcn_readlane(prow, i);
-          if (wk[k] != 0.f) {  // wave-uniform
-            const float* src = a.split_output + ((int64_t)pk * kHeads + head) * kVDim + d0;
-            if constexpr (SPLIT == 1) {
-              const f32x4 u = *(const f32x4*)src, v = *(const f32x4*)(src + 4);
+          const float wk =
+              i0 + k < n ? __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(w), min(i0 + k, 63))) : 0.f;
+          if (wk == 0.f) continue;  // a row of weight 0 may hold anything
 #pragma unroll
-              for (int j = 0; j < 4; ++j) {
-                x[k][j] = u[j];
-                x[k][4 + j] = v[j];
-              }
-            } else {
-              const f32x2 u = *(const f32x2*)src;
-              x[k][0] = u[0];
-              x[k][1] = u[1];
-            }
-          } else {
-#pragma unroll
-            for (int j = 0; j < N; ++j) x[k][j] = 0.f;
-          }
+          for (int j = 0; j < N; ++j) acc[j] += wk * x[k][j];
         }
-#pragma unroll
-        for (int k = 0; k < kBatch; ++k)
-#pragma unroll
-          for (int j = 0; j < N; ++j) acc[j] += wk[k] * x[k][j];
       }
     }
     const float inv = wsum > 0.f ? 1.f / wsum : 0.f;
@@ -891,7 +896,11 @@ __global__ __launch_bounds__(256) void mla_fp8_reduce_kernel(const pa_mla_reduce
   }
 }
 
-// Groups (query rows) up to which the reduce splits the value dims.
+// Groups (query rows) up to which the reduce splits the value dims over four
+// waves: with so few the chip idles and the chain of pieces sets the time (us,
+// one wave -> four: 4 groups 8.0 -> 6.0, 2 groups of long sequences 16.1 ->
+// 8.5).  From 17 groups the extra waves only repeat the lookup of the pieces
+// (17: 14.8 -> 15.3, 80: 15.0 -> 19.9, 128: 15.4 -> 29.1).
 constexpr int kSplitReduceGroups = 8;
 
 bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }

@@ -5152,8 +5152,8 @@ int pa_fp8_merge_balanced(const pa_fp8_stream_args* a, const void* workspace, in
   // 16 columns per wave, four loads per piece.
   // So few 16-column blocks that they leave the chip idle take the 4-column
   // form too: four times the waves and 16 pieces in flight instead of two (40
-  // pairs of 24 columns in up to 26 pieces: 17.3 -> 5.7 us; C5's 4096 blocks
-  // keep the wide one).
+  // pairs of 24 columns in up to 26 pieces: 16.8 -> 6.8 us).  With 4096
+  // blocks the wide form is the faster one (11.3 us, 26.1 with four columns).
   const int64_t blocks16 = (int64_t)a->num_seqs * a->num_kv_heads * ((eq + 15) / 16);
   const bool narrow = eq <= 4 || blocks16 <= kNarrowMergeBlocks;
   const int cols = narrow ? 4 : 16;
