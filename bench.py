@@ -207,9 +207,23 @@ def load_traffic(name: str):
 
 KERNEL_OF_ENTRY = {
     "pa_fp8_decode_partition": "pa_fp8_partition_kernel",
+    "pa_fp8_decode_split": "pa_fp8_split_kernel",
+    "pa_fp8_decode_team": "pa_fp8_team_kernel",
     "pa_fp8_decode_balanced": "pa_fp8_stream_kernel (balanced split)",
     "pa_fp8_decode_worklist": "pa_fp8_bin_kernel (work list, one workgroup per bin)",
 }
+
+
+def kernel_of(entry: str, cfg, kernels_per_step: int) -> str:
+    """Decode kernel behind a call's C entry point: a partition call of one
+    launch and at most 16 query columns runs as a split of one workgroup per pair."""
+    if entry == "pa_fp8_decode_partition":
+        if cfg.head_size != 128:
+            return "pa_fp8_generic_partition_kernel"
+        columns = cfg.query_length * cfg.num_query_heads // cfg.num_kv_heads
+        if kernels_per_step == 1 and columns <= 16:
+            return "pa_fp8_split_kernel"
+    return KERNEL_OF_ENTRY[entry]
 
 
 def flat_page_list(block_tables, ctx, block_size):
@@ -352,7 +366,7 @@ def run_config(name: str, args) -> dict:
         },
         "roofline": {
             "bound": "hbm",
-            "kernel": KERNEL_OF_ENTRY[kernel_name],
+            "kernel": kernel_of(kernel_name, cfg, kernels_per_step),
             "kernels_per_step": kernels_per_step,
             "achieved": round(achieved, 2),
             "peak": PEAK_HBM_GBPS,
