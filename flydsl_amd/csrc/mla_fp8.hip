@@ -818,7 +818,8 @@ __global__ __launch_bounds__(256) void mla_fp8_reduce_kernel(const pa_mla_reduce
   // for all of them.  The value dims depend on nothing but the rows: the first
   // kBatch pieces are loaded beside the lse, ahead of the weights (128 groups:
   // 17.3 us with the loads behind the weights, 15.4 so).  Pieces outside the split buffers or
-  // with lse -inf (no visible key) have weight 0 and are skipped.
+  // with lse -inf (no visible key) are skipped, whatever their rows hold; every other piece is
+  // added, also one whose lse is NaN or whose weight is 0, so that a NaN or an infinity shows.
   for (int row = row0; row < row1; ++row) {
     const int r = row - row0;
     float mx = kNegInf, wsum = 0.f;
@@ -859,7 +860,8 @@ __global__ __launch_bounds__(256) void mla_fp8_reduce_kernel(const pa_mla_reduce
 #pragma unroll
       for (int o = 32; o >= 1; o >>= 1) mb = fmaxf(mb, __shfl_xor(mb, o, 64));
       const float mn = fmaxf(mx, mb);
-      if (mn == kNegInf) continue;
+      const uint64_t live = __ballot(l != kNegInf);
+      if (live == 0) continue;
       const float w = l == kNegInf ? 0.f : __expf(l - mn);
       float ws = w;
 #pragma unroll
@@ -873,9 +875,8 @@ __global__ __launch_bounds__(256) void mla_fp8_reduce_kernel(const pa_mla_reduce
         if (i0 > 0) load(i0);
 #pragma unroll
         for (int k = 0; k < kBatch; ++k) {
-          const float wk =
-              i0 + k < n ? __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(w), min(i0 + k, 63))) : 0.f;
-          if (wk == 0.f) continue;  // a row of weight 0 may hold anything
+          if (!(live >> (i0 + k) & 1)) continue;  // i0 + k < 64; lanes past n are not live
+          const float wk = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(w), i0 + k));
 #pragma unroll
           for (int j = 0; j < N; ++j) acc[j] += wk * x[k][j];
         }

@@ -53,3 +53,31 @@ def test_reduce_piece_counts(groups):
         assert np.all(np.abs(got_lse[g] - want[g][1]) <= 2e-5 + 1e-5 * np.abs(want[g][1])), g
     if groups == 9:
         assert np.all(got[8] == 0) and np.all(np.isneginf(got_lse[8]))
+
+
+@pytest.mark.parametrize("groups", [2, 9])
+def test_reduce_shows_nan_and_infinity(groups):
+    """Every piece with an lse other than -inf takes part: a (row, head) whose
+    lse are NaN, alone or beside -inf, and one whose weightless piece (its lse
+    140 below the other's: exp(-140) is 0 in float32) holds NaN or an infinity come out
+    as NaN; the other heads as without them."""
+    pieces = 3
+    rng = np.random.default_rng(groups)
+    so = rng.standard_normal((groups * pieces, 1, 128, 512)).astype(np.float32)
+    sl = rng.uniform(-8, 8, (groups * pieces, 1, 128, 1)).astype(np.float32)
+    sl[:, 0, 1:5] = 0.0
+    sl[:3, 0, 1] = np.nan  # every piece
+    sl[:3, 0, 2] = [[np.nan], [-np.inf], [-np.inf]]
+    sl[1, 0, 3:5] = -140.0
+    so[1, 0, 3, 7], so[1, 0, 4, 8] = np.nan, np.inf
+    dev = lambda x: torch.from_numpy(x).cuda()  # noqa: E731
+    args = [dev(np.arange(0, groups * pieces + 1, pieces, dtype=np.int32)),
+            dev(np.array([[g, g + 1] for g in range(groups)], np.int32)),
+            dev(np.arange(groups * pieces, dtype=np.int32))]
+    out = torch.zeros((groups, 128, 512), dtype=torch.bfloat16, device="cuda")
+    mla_reduce_v1(dev(so), dev(sl), *args, 1, out)
+    bad = torch.isnan(out).cpu()
+    want = torch.zeros_like(bad)
+    want[0, 1:3] = True
+    want[0, 3, 7] = want[0, 4, 8] = True
+    assert torch.equal(bad, want)
