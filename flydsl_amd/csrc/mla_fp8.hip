@@ -794,6 +794,28 @@ __global__ __launch_bounds__(Shape<NHT>::threads, 1) void mla_fp8_decode_kernel(
   }
 }
 
+// Reductions over the wave: rows of 16 lanes by DPP (quad swaps, then the 8-
+// and 16-lane mirrors), then across the rows.  (Twelve `__shfl_xor` are as many
+// LDS round trips, 0.3 us of a 3.4 us reduce of two pieces.)
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false));
+}
+__device__ __forceinline__ float wave_max(float v) {
+  v = fmaxf(v, dpp<0xB1>(v));
+  v = fmaxf(v, dpp<0x4E>(v));
+  v = fmaxf(v, dpp<0x141>(v));
+  v = fmaxf(v, dpp<0x140>(v));
+  return max_over_groups(v);
+}
+__device__ __forceinline__ float wave_sum(float v) {
+  v += dpp<0xB1>(v);
+  v += dpp<0x4E>(v);
+  v += dpp<0x141>(v);
+  v += dpp<0x140>(v);
+  return sum_over_groups(v);
+}
+
 // One wave per (group, head, 512 / SPLIT value dims): lane l merges 8 / SPLIT
 // of them.  SPLIT = 4 where the heads alone are too few waves for the chip
 // (4 rows x 128 heads): four times the waves, each with twice the pieces in
@@ -816,8 +838,8 @@ __global__ __launch_bounds__(256) void mla_fp8_reduce_kernel(const pa_mla_reduce
   const int row1 = min(max(a.reduce_final_map[2 * gidx + 1], row0), a.num_rows);
   // Lane i takes piece i's row and lse, 64 pieces at a time: two round trips
   // for all of them.  The value dims depend on nothing but the rows: the first
-  // kBatch pieces are loaded beside the lse, ahead of the weights (128 groups:
-  // 17.3 us with the loads behind the weights, 15.4 so).  Pieces outside the split buffers or
+  // kBatch pieces are loaded beside the lse, ahead of the weights (128 groups
+  // of 2 pieces: 2 us less than with the loads behind the weights).  Pieces outside the split buffers or
   // with lse -inf (no visible key) are skipped, whatever their rows hold; every other piece is
   // added, also one whose lse is NaN or whose weight is 0, so that a NaN or an infinity shows.
   for (int row = row0; row < row1; ++row) {
@@ -856,18 +878,12 @@ __global__ __launch_bounds__(256) void mla_fp8_reduce_kernel(const pa_mla_reduce
         }
       };
       load(0);
-      float mb = l;
-#pragma unroll
-      for (int o = 32; o >= 1; o >>= 1) mb = fmaxf(mb, __shfl_xor(mb, o, 64));
-      const float mn = fmaxf(mx, mb);
+      const float mn = fmaxf(mx, wave_max(l));
       const uint64_t live = __ballot(l != kNegInf);
       if (live == 0) continue;
       const float w = l == kNegInf ? 0.f : __expf(l - mn);
-      float ws = w;
-#pragma unroll
-      for (int o = 32; o >= 1; o >>= 1) ws += __shfl_xor(ws, o, 64);
       const float fold = mx == kNegInf ? 0.f : __expf(mx - mn);
-      wsum = wsum * fold + ws;
+      wsum = wsum * fold + wave_sum(w);
 #pragma unroll
       for (int j = 0; j < N; ++j) acc[j] *= fold;
       mx = mn;
@@ -899,9 +915,11 @@ __global__ __launch_bounds__(256) void mla_fp8_reduce_kernel(const pa_mla_reduce
 
 // Groups (query rows) up to which the reduce splits the value dims over four
 // waves: with so few the chip idles and the chain of pieces sets the time (us,
-// one wave -> four: 4 groups 8.0 -> 6.0, 2 groups of long sequences 16.1 ->
-// 8.5).  From 17 groups the extra waves only repeat the lookup of the pieces
-// (17: 14.8 -> 15.3, 80: 15.0 -> 19.9, 128: 15.4 -> 29.1).
+// one wave -> four: 4 groups of 16 pieces 5.9 -> 4.1, 2 of 64 19 -> 8.1, 8 of 16 7.0 -> 6.0).  Past
+// 4 groups only for more than 8 pieces a group: with fewer the four times as
+// many workgroups cost more than they hide (8 groups of 2: 3.3 -> 3.7).  With
+// many groups the extra waves only repeat the lookup of the pieces (80 groups:
+// 15.0 -> 19.9, 128: 15.4 -> 29.1).
 constexpr int kSplitReduceGroups = 8;
 
 bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
@@ -1023,7 +1041,7 @@ extern "C" int pa_fp8_mla_reduce(const pa_mla_reduce_args* a, void* stream) {
   if (a->num_partial > 0 && (!a->split_output || !a->split_lse || !a->reduce_partial_map)) return PA_ERR_NULL_ARG;
   if (!aligned16(a->final_output) || (a->split_output && !aligned16(a->split_output))) return PA_ERR_ALIGN;
   hipStream_t s = (hipStream_t)stream;
-  if (a->num_groups <= kSplitReduceGroups)
+  if (a->num_groups <= 4 || (a->num_groups <= kSplitReduceGroups && a->num_partial > 8 * a->num_groups))
     hipLaunchKernelGGL(mla_fp8_reduce_kernel<4>, dim3(a->num_groups, kHeads), dim3(256), 0, s, *a);
   else
     hipLaunchKernelGGL(mla_fp8_reduce_kernel<1>, dim3(a->num_groups, kHeads / 4), dim3(256), 0, s, *a);

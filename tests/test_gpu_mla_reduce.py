@@ -1,5 +1,5 @@
 """The MLA reduce alone against the oracle's merge, at the edges of its forms:
-8 and 9 groups (value dims over four waves or one), piece counts around the 8
+8 and 9 groups (value dims over four waves or one; 6 groups of few pieces: one), piece counts around the 8
 and 16 in flight and the 64 a wave looks up at a time, pieces with lse -inf
 whose rows hold NaN, and a group whose pieces are all such.
 
@@ -55,7 +55,7 @@ def test_reduce_piece_counts(groups):
         assert np.all(got[8] == 0) and np.all(np.isneginf(got_lse[8]))
 
 
-@pytest.mark.parametrize("groups", [2, 9])
+@pytest.mark.parametrize("groups", [2, 6, 9])
 def test_reduce_shows_nan_and_infinity(groups):
     """Every piece with an lse other than -inf takes part: a (row, head) whose
     lse are NaN, alone or beside -inf, and one whose weightless piece (its lse
