@@ -289,44 +289,62 @@ def _stream_ok(route: str, batch: int, eqgs: int, user_partials: bool, owner: bo
 # Split decode: workgroups a pair is spread over.  As many as keep the launch
 # to one workgroup per CU (a part-filled second round costs a whole share),
 # up to SPLIT_MAX of them with at least SPLIT_CHUNKS chunks each at full
-# length; more, up to SPLIT_MOST workgroups in all, when a share would exceed
-# SPLIT_SHARE chunks.  Measured (us per call, page 16): 8 pairs of 512 tokens
+# length.  Measured (us per call, page 16): 8 pairs of 512 tokens
 # 19.2 on the two-kernel schedules -> 6.8 with one workgroup per pair; of 8192
-# tokens 21.4 -> 13.0 with 8 (26.6 with 2, 13.1 with 16); 128 pairs of 8192
-# tokens 52.5 -> 45.8 with 2 (52.0 with 1, 49.7 with 4); 16 pairs of 8192 ..
+# tokens 21.4 -> 13.0 with 8 (26.6 with 2, 13.1 with 16); 16 pairs of 8192 ..
 # 32768 tokens 37.2 -> 24.6 with 16 (28.9 with 8, 32.9 with 20: 320 workgroups).
-# Beyond SPLIT_SHARE the longest sequence's share sets the time of a ragged
-# batch (512 pairs of 1024 .. 16384 tokens: 213 with one) and equal runs over
-# the whole batch are the better schedule.
 SPLIT_CHUNKS = 16
 SPLIT_MAX = 32
 SPLIT_SHARE = 256
 SPLIT_MOST = 1024
-SPLIT_EVEN = 128
 SPLIT_FEW = 64
 SPLIT_MAX_SEQS = 65535  # a grid dimension
 
 
-def _split_count(pairs: int, capacity_chunks: int, num_cu: int, bounded: bool = False) -> int:
+def _longest_share(pairs: int, s: int, num_cu: int, columns: int) -> int:
+    """Chunks a workgroup may get at full length, with ``s`` per pair, before
+    equal runs over the whole batch (balanced up to BALANCED_MAX_COLUMNS
+    columns, else team) are the better schedule: the longest sequence's share
+    sets the time of a split decode, and the more so the fewer workgroups the
+    other sequences leave to it.  Percent of the balanced split's time, lengths
+    equal / uniform / lognormal up to the capacity, on both sides of each line
+    (4 columns): 112 pairs of 8192 tokens (2 workgroups, 128 chunks) 82 / 98 /
+    88, 96 pairs 80 / 102 / 119; 96 to 128 of 16384 tokens 87..95 / 105..122 /
+    107..138; 64 pairs of 32768 tokens (4, 256) 90 / 100 / 100, of 65536 95 / 112 /
+    135; 32 of 131072 (8, 512) 92 / 101 / 107, of 262144 98 / 112 / 141.  One
+    workgroup per pair: 160 to 256 pairs of 4096 tokens 79..88 / 88..97 / 94..113; 136,
+    which leave half of the CUs idle, 87..97 / 110..122 / 99..102, but of 3072
+    81 / 90 / 91; 272 to 384, which leave as much of a second round, 90..115 /
+    101..120 / 91..118, of 2048 81..100 / 80..92 / 65..76.
+    With 5 to 16 columns the team runs gain less, in percent of the slot
+    schedule's time: 96 pairs of 8192 tokens split 78 / 79 / 89, team 98 / 90 /
+    97; of 16384 86 / 101 / 125 and 101 / 90 / 89.  Few pairs: 64 of 65536 tokens 95 /
+    93 / 121 and 102 / 83 / 67, but a table that wide with contexts up to 4096 in it
+    56 and 119."""
+    few = pairs <= SPLIT_FEW
+    if columns > BALANCED_MAX_COLUMNS:
+        return 128 if s == 1 else (256 if few else 80) * s
+    if s > 1:
+        return 64 * s
+    if pairs <= num_cu:
+        return 128 if 8 * pairs >= 5 * num_cu else 96
+    return 128 if 4 * pairs >= 7 * num_cu else 64
+
+
+def _split_count(pairs: int, capacity_chunks: int, num_cu: int, bounded: bool = False, columns: int = 16) -> int:
     """Workgroups per (sequence, kv head) pair of a split decode over ``pairs``
-    pairs of at most ``capacity_chunks`` 32-token chunks each (``bounded``: by
-    a window, so that they hardly differ); 0 when the split decode is not the
-    schedule for them."""
-    s = min(SPLIT_MAX, max(1, num_cu // pairs))
+    pairs of at most ``capacity_chunks`` 32-token chunks and ``columns`` query
+    columns each (``bounded``: by a window, so that they hardly differ); 0 when
+    the split decode is not the schedule for them."""
+    long = _cdiv(capacity_chunks, SPLIT_SHARE)
+    s = min(max(SPLIT_MAX, long), max(1, num_cu // pairs))
     s = max(1, min(s, _cdiv(capacity_chunks, SPLIT_CHUNKS)))
-    s = max(s, _cdiv(capacity_chunks, SPLIT_SHARE))
-    if not bounded and capacity_chunks > SPLIT_EVEN:
-        # Uneven pairs, each a large part of a CU's work: in more workgroups
-        # than CUs, or one to a CU where the longest takes twice the mean,
-        # equal runs are faster (212 pairs, lognormal up to 9970 tokens: 43.0
-        # us balanced, 50.5 with 2; 200 pairs up to 8192, 16 columns: 42.2
-        # with 1, team runs 32.7).  Few pairs still gain from one launch (64
-        # pairs of 4096 .. 32768 tokens: 75.7 balanced, 69.7 with 4).
-        if s > 1 and pairs > SPLIT_FEW and pairs * s > num_cu:
-            return 0
-        if s == 1 and num_cu // 2 < pairs < 2 * num_cu:
-            return 0
-    return s if s == 1 or pairs * s <= SPLIT_MOST else 0
+    if bounded:
+        s = max(s, long)
+        return s if s == 1 or pairs * s <= SPLIT_MOST else 0
+    # two pairs and more for every CU: any schedule fills the chip
+    most = SPLIT_SHARE if pairs >= 2 * num_cu else _longest_share(pairs, s, num_cu, columns)
+    return s if _cdiv(capacity_chunks, s) <= most else 0
 
 
 def _stream_layout_ok(output, key_cache, value_cache, key_scale, per_token_kv: bool) -> bool:
@@ -367,7 +385,11 @@ def _plan(route: str, batch: int, kv_heads: int, P: int, eqgs: int, head_size: i
     balanced = False if generic else _balanced_ok(route, batch, eqgs, user_partials, owner)
     if balanced == _SPLIT:
         if one_launch:
-            splits = _split_count(batch * kv_heads, max(1, _cdiv(tokens, 32)), _cu_count(dev), route == "sw")
+            # (a flat page list gives the whole batch's pages: four times the
+            # mean stands for the longest sequence)
+            if capacity is None:
+                tokens = min(tokens, 4 * _cdiv(tokens, batch))
+            splits = _split_count(batch * kv_heads, max(1, _cdiv(tokens, 32)), _cu_count(dev), route == "sw", eqgs)
             if splits == 1:
                 return OWNER, P, P
             if splits > 1:

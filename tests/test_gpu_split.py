@@ -108,9 +108,19 @@ def test_split_counts():
     assert pd._split_count(8, 2, 256) == 1 and pd._split_count(8, 16, 256) == 1  # short: one workgroup per pair
     assert pd._split_count(8, 256, 256) == 16 and pd._split_count(128, 256, 256) == 2
     assert pd._split_count(512, 128, 256) == 1 and pd._split_count(56, 824, 256) == 4
-    assert pd._split_count(32, 4096, 256) == 16  # shares of at most 256 chunks
+    assert pd._split_count(32, 4096, 256) == 8  # one round of workgroups
     # uneven pairs that are large parts of a CU's work: equal runs, unless few
     assert pd._split_count(212, 312, 256) == 0 and pd._split_count(200, 256, 256) == 0
     assert pd._split_count(200, 256, 256, True) == 1 and pd._split_count(200, 128, 256) == 1
     assert pd._split_count(64, 975, 256) == 4
     assert pd._split_count(1024, 1024, 256) == 0  # many long pairs: equal runs over the batch
+    # where the longest sequence's share would set the time: both sides of the lines
+    for pairs, chunks, columns, s in ((96, 256, 4, 2), (96, 257, 4, 0), (64, 1024, 4, 4), (64, 1025, 4, 0), (33, 3136, 4, 7),
+                                      (33, 3137, 4, 0), (136, 96, 4, 1), (136, 97, 4, 0), (160, 128, 4, 1),
+                                      (256, 129, 4, 0), (257, 64, 4, 1), (257, 65, 4, 0), (448, 128, 4, 1),
+                                      (136, 128, 5, 1), (272, 129, 16, 0), (96, 320, 16, 2), (96, 321, 16, 0),
+                                      (64, 4096, 16, 4), (64, 4097, 16, 0), (1, 16384, 4, 64)):
+        assert pd._split_count(pairs, chunks, 256, False, columns) == s, (pairs, chunks, columns)
+    # a flat page list gives the batch's total: its mean counts
+    plan = lambda tokens: pd._plan("flat", 64, 2, 0, 8, 128, 128, None, tokens, False, False, False, True, False, 0)
+    assert plan(64 * 512)[0] == "split" and plan(64 * 8192)[0] == "team"
