@@ -2300,8 +2300,14 @@ __global__ __launch_bounds__(64 * kBinWaves) void pa_fp8_bin_kernel(
 //  * the s workgroups of a pair leave their folded states in workspace slots
 //    with agent-scope stores (written through the XCD's own L2), count
 //    themselves in the pair's counter once the stores have retired, and the
-//    last one folds the slots, read with agent-scope loads.  It resets the
-//    counter, so counters that are zero before a launch are zero after it.
+//    last one folds the slots, read with agent-scope loads.  The count wraps to
+//    zero at s, so counters that are zero before a launch are zero after it,
+//    and after two that overlap (each may then fold the other's states, but
+//    the launches behind them count from zero again; a count and a separate
+//    store of zero lose one another's arrivals).
+//    Counting the workgroups without a share as well, or the whole grid, would also
+//    outlast lengths that change during a launch; it took 0.1 to 1 us of a
+//    10 us call, 1 to 2.6 us of a team call.
 //    Nothing waits for another workgroup, and there is no release fence
 //    (whose L2 write-back costs more than the second kernel).
 //
@@ -2501,11 +2507,7 @@ __global__ __launch_bounds__(64 * WAVES) void pa_fp8_split_kernel(
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   LDS_AS int* flag = (LDS_AS int*)((LDS_AS unsigned char*)smem + W * kWaveBytes);
-  if (tid == 0) {
-    const int old = __hip_atomic_fetch_add(&counters[pair], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    *flag = old == s - 1;
-    if (old == s - 1) __hip_atomic_store(&counters[pair], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
+  if (tid == 0) *flag = atomicInc((unsigned*)&counters[pair], (unsigned)(s - 1)) >= (unsigned)(s - 1);
   __syncthreads();
   if (__builtin_amdgcn_readfirstlane(*flag) == 0) return;
   constexpr int kBatch = W == 8 ? 8 : 4;  // slots whose loads are in flight together
@@ -2976,13 +2978,12 @@ __global__ __launch_bounds__(64 * kTeamWaves) void pa_fp8_team_kernel(
     }
     st_agent(s + 8192 + lane * 8, pack_f32x2(M, L));
     const int rf = pa_plan_run_of_chunk(q0, T, nw);
-    const int pieces = pa_plan_run_of_chunk(q0 + p.nb - 1, T, nw) - rf + 1;
+    // (clamped: nb may be a later reading of the length than T)
+    const int pieces = pa_min(pa_plan_run_of_chunk(q0 + p.nb - 1, T, nw), nw - 1) - rf + 1;
     // The state is out before the count says so.
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     if (lane == 0) {
-      const int old = __hip_atomic_fetch_add(&counters[(int64_t)p.b * H + p.h], 1, __ATOMIC_RELAXED,
-                                             __HIP_MEMORY_SCOPE_AGENT);
-      if (old == pieces - 1) {
+      if (atomicInc((unsigned*)&counters[(int64_t)p.b * H + p.h], (unsigned)(pieces - 1)) >= (unsigned)(pieces - 1)) {
         flags[4 * side] = pieces;
         flags[4 * side + 1] = rf;
         flags[4 * side + 2] = p.b;
@@ -3048,8 +3049,6 @@ __global__ __launch_bounds__(64 * kTeamWaves) void pa_fp8_team_kernel(
         for (int j = 0; j < 8; ++j) acc[j] += *(const LDS_AS f32x4*)(f + j * 1024 + lane * 16) * fr;
       }
       store_piece<true>(a, output, nullptr, nullptr, p, acc, Lc, Mc, 1.0f, c16, grp);
-      if (lane == 0)
-        __hip_atomic_store(&counters[(int64_t)p.b * H + p.h], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     __syncthreads();
   }

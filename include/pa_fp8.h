@@ -298,8 +298,10 @@ int64_t pa_fp8_static_scratch_bytes(void);
  * short sequences), the last of which merges them.  With num_workers > 1 it
  * needs `slots` (pa_fp8_split_slot_bytes() bytes, contents irrelevant) and
  * `counters` (one int32 per (sequence, kv head), zero before the first
- * launch; every launch leaves them zero); launches that may run at the same
- * time need buffers of their own.  Arguments and checks as
+ * launch; every launch leaves them zero).  Launches that may run at the same
+ * time need buffers of their own (launches that overlap all the same may be
+ * wrong, those behind them are not).  context_lengths must not change during a
+ * launch: the counters may then have to be cleared again.  Arguments and checks as
  * pa_fp8_decode_balanced; PA_ERR_GROUP above 16 columns, PA_ERR_SHAPE above
  * 65535 sequences or splits.
  */
@@ -313,8 +315,8 @@ int pa_fp8_decode_split(const pa_fp8_stream_args* args, void* slots, int64_t slo
  * Pairs cut between workgroups are merged by the workgroup that finishes
  * them last, through `slots` (pa_fp8_team_slot_bytes(num_workers) bytes,
  * contents irrelevant) and `counters` (one int32 per (sequence, kv head),
- * zero before the first launch; every launch leaves them zero).  Launches
- * that may run at the same time need buffers of their own.  Same arguments,
+ * zero before the first launch; every launch leaves them zero); overlapping
+ * launches and changing lengths as for pa_fp8_decode_split.  Same arguments,
  * limits and checks as pa_fp8_decode_balanced; PA_ERR_GROUP above 16 columns.
  */
 int64_t pa_fp8_team_slot_bytes(int num_workers);

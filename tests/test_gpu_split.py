@@ -104,6 +104,47 @@ def test_launcher_shares_one_workspace_per_stream():
     assert len(pd._workspaces) <= pd._WORKSPACES_KEPT
 
 
+def launcher(case, S, team, counters):
+    """launch(out, stream) of one call with a workspace of its own."""
+    a = pd._stream_args(case["query"], case["query"], case["key_cache"], case["value_cache"], case["context_lengths"],
+                        case["block_tables"], None, case["softmax_scale"], case["key_scale"], case["value_scale"],
+                        case["key_scale"].dim() > 1, True, "bf16", _lib.DTYPE_BF16, case["sliding_window"])
+    a.num_workers = S
+    slots = torch.empty(_lib.team_slot_bytes(S) if team else _lib.split_slot_bytes(a.num_seqs, a.num_kv_heads, S),
+                        dtype=torch.uint8, device=DEV)
+    entry = _lib.load().pa_fp8_decode_team if team else _lib.load().pa_fp8_decode_split
+
+    def launch(out, stream):
+        a.output = out.data_ptr()
+        _lib.check(entry(ctypes.byref(a), slots.data_ptr(), slots.numel(), counters.data_ptr(), counters.numel(),
+                         ctypes.c_void_p(stream.cuda_stream)), "decode")
+    return launch
+
+
+RAGGED = dict(batch=6, num_query_heads=16, num_kv_heads=2, ctx=[9000, 17, 3000, 0, 700, 5000])
+
+
+@pytest.mark.parametrize("team", [False, True])
+def test_overlapping_launches_leave_the_workspace_sound(team):
+    """Launches of one workspace that overlap may be wrong; one after them is
+    right and finds every counter zero."""
+    case = to_dev(make_case(seed=8, **RAGGED))
+    counters = torch.zeros(12, dtype=torch.int32, device=DEV)
+    launch = launcher(case, 64 if team else 8, team, counters)
+    want = torch.empty_like(case["query"])
+    launch(want, torch.cuda.current_stream())
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    outs = [torch.empty_like(want) for _ in range(2)]
+    torch.cuda.synchronize()
+    for _ in range(50):
+        for out, s in zip(outs, streams):
+            launch(out, s)
+    torch.cuda.synchronize()
+    assert bool((counters == 0).all())
+    launch(outs[0], torch.cuda.current_stream())
+    assert torch.equal(outs[0], want)
+
+
 def test_split_counts():
     assert pd._split_count(8, 2, 256) == 1 and pd._split_count(8, 16, 256) == 1  # short: one workgroup per pair
     assert pd._split_count(8, 256, 256) == 16 and pd._split_count(128, 256, 256) == 2
