@@ -438,9 +438,15 @@ _workspaces_lock = threading.Lock()
 def _native_workspace(index: int, stream_id: int, pairs: int, nbytes: int):
     """Pointers of the workspace of the current stream ``stream_id`` of device
     ``index``, and the workspace itself for the caller to hold."""
-    ws = _workspaces.get((index, stream_id))
+    key = (index, stream_id)
+    ws = _workspaces.get(key)
     if ws is None or ws.slots.numel() < nbytes or ws.counters.numel() < pairs:
         ws = _split_workspace(index, torch.cuda.current_stream(index), pairs, nbytes, True)
+    else:
+        try:
+            _workspaces.move_to_end(key)
+        except KeyError:  # another thread has just dropped it; this call holds it
+            pass
     return ws.pointers() + (ws,)
 
 
