@@ -2,7 +2,8 @@
 head) over up to S workgroups, merged by the last one) and of the team decode
 (pa_fp8_decode_team: equal runs of the batch per workgroup).  Edges of its ranges:
 contexts around a chunk, a share and a split, empty sequences, 1 to 16 query
-columns, both kernels' wave counts, windows, the flat page list."""
+columns, both kernels' wave counts, windows, the flat page list with sequences
+that have no pages; and of the workspaces that the launchers give them."""
 
 from __future__ import annotations
 
@@ -104,14 +105,16 @@ def test_launcher_shares_one_workspace_per_stream():
     assert len(pd._workspaces) <= pd._WORKSPACES_KEPT
 
 
-def launcher(case, S, team, counters):
-    """launch(out, stream) of one call with a workspace of its own."""
+def launcher(case, S, team, counters, pages=None, indptr=None):
+    """launch(out, stream) of one call with a workspace of its own (``pages``,
+    ``indptr``: a flat page list in the place of the block table)."""
     a = pd._stream_args(case["query"], case["query"], case["key_cache"], case["value_cache"], case["context_lengths"],
-                        case["block_tables"], None, case["softmax_scale"], case["key_scale"], case["value_scale"],
-                        case["key_scale"].dim() > 1, True, "bf16", _lib.DTYPE_BF16, case["sliding_window"])
+                        case["block_tables"] if pages is None else pages, indptr, case["softmax_scale"],
+                        case["key_scale"], case["value_scale"], case["key_scale"].dim() > 1, True, "bf16",
+                        _lib.DTYPE_BF16, case["sliding_window"])
     a.num_workers = S
-    slots = torch.empty(_lib.team_slot_bytes(S) if team else _lib.split_slot_bytes(a.num_seqs, a.num_kv_heads, S),
-                        dtype=torch.uint8, device=DEV)
+    nbytes = _lib.team_slot_bytes(S) if team else _lib.split_slot_bytes(a.num_seqs, a.num_kv_heads, S)
+    slots = torch.full((max(16, nbytes),), 0xFF, dtype=torch.uint8, device=DEV)
     entry = _lib.load().pa_fp8_decode_team if team else _lib.load().pa_fp8_decode_split
 
     def launch(out, stream):
@@ -119,6 +122,62 @@ def launcher(case, S, team, counters):
         _lib.check(entry(ctypes.byref(a), slots.data_ptr(), slots.numel(), counters.data_ptr(), counters.numel(),
                          ctypes.c_void_p(stream.cuda_stream)), "decode")
     return launch
+
+
+@pytest.mark.parametrize("kernel,workers", [("split", 1), ("split", 8), ("team", 5), ("team", 256)])
+@pytest.mark.parametrize("block_size,per_token", [(16, True), (128, False), (1024, True)])
+def test_flat_page_list(kernel, workers, block_size, per_token):
+    """Pages of all sequences end to end, two sequences without any (one of
+    them with a length all the same): those rows are zero."""
+    ctx = [700, 0, 3000, 1, 500, 6000, 33]
+    case = make_case(batch=7, num_query_heads=24, num_kv_heads=2, block_size=block_size, ctx=ctx, per_token=per_token,
+                     seed=workers)
+    ref = torch_oracle(dict(case, context_lengths=case["context_lengths"].clamp(min=1)), float_out=False)
+    none = (1, 4)
+    for b in none:
+        ref[b] = 0
+    case = to_dev(case)
+    rows = [case["block_tables"][b, : 0 if b in none else -(-c // block_size)] for b, c in enumerate(ctx)]
+    pages = torch.cat(rows)
+    indptr = torch.tensor([0] + [len(r) for r in rows]).cumsum(0).to(torch.int32).to(DEV)
+    counters = torch.zeros(14, dtype=torch.int32, device=DEV)
+    out = torch.empty_like(case["query"])
+    launcher(case, workers, kernel == "team", counters, pages, indptr)(out, torch.cuda.current_stream())
+    assert bool((counters == 0).all())
+    assert_parity(out, ref, f"{kernel}/{workers}/{block_size}")
+
+
+@pytest.mark.parametrize("workgroups", [1, 5, 64, 256])
+@pytest.mark.parametrize("ql", [1, 2])
+def test_team_window(ql, workgroups):
+    case = make_case(batch=7, query_length=ql, num_query_heads=16, num_kv_heads=2, ctx=[5, 300, 1500, 6000, 1001, 2033, 64],
+                     sliding_window=1000, seed=workgroups)
+    ref = torch_oracle(case, float_out=False)
+    assert_parity(split(to_dev(case), workgroups, team=True), ref, f"window/{ql}/{workgroups}")
+
+
+@pytest.mark.parametrize("gqa", [4, 16])
+def test_native_workspaces_of_overlapping_streams(gqa):
+    """Calls on the current stream of two unordered streams, and on a stream
+    that torch does not own, by the native path (no ``stream``)."""
+    case = to_dev(make_case(batch=2, ctx=[3000, 9000], num_query_heads=2 * gqa, seed=5))
+    ref = torch_oracle({k: (v.cpu() if isinstance(v, torch.Tensor) else v) for k, v in case.items()}, float_out=False)
+    args = (case["query"], case["key_cache"], case["value_cache"], case["context_lengths"], None, None,
+            case["softmax_scale"], case["key_scale"], case["value_scale"])
+    own = torch.cuda.Stream()
+    streams = [torch.cuda.Stream(), torch.cuda.Stream(), torch.cuda.ExternalStream(own.cuda_stream)]
+    outs = [torch.empty_like(case["query"]) for _ in range(30)]
+    torch.cuda.synchronize()
+    for i, out in enumerate(outs):
+        with torch.cuda.stream(streams[i % 3]):
+            pa_decode_ps_launch(out, *args, block_tables=case["block_tables"])
+    torch.cuda.synchronize()
+    for out in outs:
+        assert torch.equal(out, outs[0])
+    assert_parity(outs[0], ref, "three streams")
+    kept = [pd._workspaces[0, s.stream_id] for s in streams[:2]]
+    assert kept[0] is not kept[1] and (0, streams[2].stream_id) not in pd._workspaces
+    assert all(int(w.counters.abs().sum()) == 0 for w in kept)
 
 
 RAGGED = dict(batch=6, num_query_heads=16, num_kv_heads=2, ctx=[9000, 17, 3000, 0, 700, 5000])
