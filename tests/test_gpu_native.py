@@ -193,3 +193,66 @@ def test_forms_left_to_python():
         assert _lib.native().pa_decode(*args) is None  # under capture
     torch.cuda.synchronize()
     assert bool((out == 5.0).all())
+
+
+def refused(call, args, changes):
+    """Every single change of ``args`` comes back as None, unlaunched."""
+    for i, x in changes:
+        a = list(args)
+        a[i] = x
+        assert call(*a) is None, (i, x)
+
+
+class Subclass(torch.Tensor):
+    pass
+
+
+def test_rope_forms_left_to_python():
+    T, qh, kh, d, bs, nb = 5, 4, 2, 64, 16, 4
+    bf = lambda *s: torch.ones(*s, dtype=torch.bfloat16, device=DEV)
+    kc, vc = (torch.full(s, 7, dtype=torch.uint8, device=DEV) for s in ((nb, kh, d // 16, bs, 16), (nb, kh, d, bs)))
+    qo, ko = bf(T, qh, d) * 5, bf(T, kh, d) * 5
+    pos = torch.arange(T, dtype=torch.int32, device=DEV)
+    one = torch.ones(1, device=DEV)
+    args = [(d, qh, kh, bs, 0, 1, 1, 1, 0), bf(T, qh, d), bf(T, kh, d), bf(T, kh, d), pos, bf(9, d // 2), bf(9, d // 2),
+            pos.clone(), kc, vc, qo, ko, T, one, one.clone()]
+    refused(_lib.native().rope, args, [
+        (1, bf(T, qh, 2 * d)[..., ::2]), (1, bf(T + 1, qh, d)), (1, bf(T, qh, d).half()), (1, bf(T, qh, d).as_subclass(Subclass)),
+        (2, bf(T, kh, d).cpu()), (3, bf(T, kh + 1, d)), (4, pos.long()), (4, pos[:-1]), (5, bf(9, d)), (6, bf(8, d // 2)),
+        (7, pos.view(1, -1)), (8, kc.to(torch.bfloat16)), (8, kc.transpose(0, 1)), (9, vc[:, :, :, :8]),
+        (9, vc.view(nb, kh, 1, d, bs)[:-1]), (10, qo.half()), (11, bf(T, kh, d, 1)), (12, T - 1), (12, 0), (12, float(T)),
+        (13, None), (13, one.double()), (14, one[:0])])
+    assert bool((kc == 7).all()) and bool((vc == 7).all()) and bool((qo == 5).all()) and bool((ko == 5).all())
+
+
+def test_qknr_forms_left_to_python():
+    T, h, d, rd = 5, 2, 128, 64
+    bf = lambda *s: torch.ones(*s, dtype=torch.bfloat16, device=DEV)
+    pos = torch.zeros(T, dtype=torch.int64, device=DEV)
+    args = [bf(T, h * d), bf(T, d), bf(d), bf(9, rd // 2), bf(9, rd // 2), pos, h, d, rd, None, True, 64, 0]
+    refused(_lib.native().qknr, args, [
+        (0, bf(T, h * d).half()), (0, bf(T, h * d + 1)[:, 1:]), (0, bf(T, d, h).transpose(1, 2)), (0, bf(0, h * d)),
+        (0, bf(T, h * d).as_subclass(Subclass)), (1, bf(T - 1, d)), (1, bf(T, d + 1)[:, :d]), (1, bf(T, d).cpu()), (2, bf(d + 1)),
+        (2, bf(2 * d)[::2]), (3, bf(9, rd)), (4, bf(8, rd // 2)), (4, bf(9, rd // 2).float()), (5, pos.int()), (5, pos[:-1]),
+        (6, h + 1), (9, bf(d).float()), (9, bf(d - 1)), (11, 48), (11, 0)])
+
+
+def test_mla_forms_left_to_python():
+    fp8 = lambda *s: torch.zeros(*s, dtype=torch.uint8, device=DEV).view(torch.float8_e4m3fn)
+    i32 = lambda *s: torch.zeros(*s, dtype=torch.int32, device=DEV)
+    R, n = 2, 3
+    out = torch.full((R, 128, 512), 5.0, dtype=torch.bfloat16, device=DEV)
+    so, sl = torch.zeros(n, 1, 128, 512, device=DEV), torch.zeros(n, 1, 128, 1, device=DEV)
+    args = [fp8(R, 128, 576), fp8(9, 1, 1, 576), i32(9), i32(3), i32(2, 8), out, so, sl, 0.05, False]
+    refused(_lib.native().mla_decode, args, [
+        (0, fp8(R, 64, 576)), (0, fp8(R, 128, 576).view(torch.uint8)), (0, fp8(R, 128, 576).view(torch.float8_e4m3fnuz)),
+        (0, fp8(0, 128, 576)), (1, fp8(9, 2, 1, 576)), (1, fp8(9, 1, 576)), (1, fp8(9, 1, 1, 576).cpu()), (2, i32(9).long()),
+        (2, i32(18)[::2]), (3, i32(0)), (4, i32(2, 8).float()), (5, out.float()), (5, out[:1]), (5, out.transpose(0, 1)),
+        (6, so.half()), (6, so[:2]), (7, sl[..., 0]), (8, 1), (0, fp8(R, 128, 576).as_subclass(Subclass))])
+    args = [so, sl, i32(R + 1), i32(R, 2), i32(n), out]
+    refused(_lib.native().mla_reduce, args, [
+        (0, so.double()), (0, so.transpose(0, 2)), (1, sl.cpu()), (2, i32(R + 1).long()), (2, i32(0)), (2, i32(R + 2)),
+        (3, i32(R, 4)[:, ::2]), (4, i32(n).short()), (5, out.half()), (5, out[..., :256].contiguous()),
+        (5, out.transpose(0, 1))])
+    torch.cuda.synchronize()
+    assert bool((out == 5.0).all())
