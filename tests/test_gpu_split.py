@@ -180,6 +180,33 @@ def test_native_workspaces_of_overlapping_streams(gqa):
     assert all(int(w.counters.abs().sum()) == 0 for w in kept)
 
 
+@pytest.mark.parametrize("name", ["split", "team"])
+def test_prepared_calls_replay_from_a_graph(name):
+    """A prepared call's launches, captured: every replay gives the eager
+    call's bits, with eager decodes on the stream in between."""
+    shape = {"split": dict(batch=2, ctx=[3000, 9000], num_query_heads=16),
+             "team": dict(batch=150, num_query_heads=64, num_kv_heads=8, ctx=[20000] + [30] * 149)}[name]
+    case = to_dev(make_case(seed=6, **shape))
+    args = (case["query"], case["key_cache"], case["value_cache"], case["context_lengths"], None, None,
+            case["softmax_scale"], case["key_scale"], case["value_scale"])
+    out, eager = torch.empty_like(case["query"]), torch.empty_like(case["query"])
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    call = pd.prepare_pa_decode(out, *args, block_tables=case["block_tables"], stream=s)
+    assert [n for n, _ in call.kernels()] == [f"pa_fp8_decode_{name}"]
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=s):
+        call.launch()
+        call.launch()
+    for _ in range(4):
+        out.zero_()
+        graph.replay()
+        pa_decode_ps_launch(eager, *args, block_tables=case["block_tables"])
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager)
+
+
 RAGGED = dict(batch=6, num_query_heads=16, num_kv_heads=2, ctx=[9000, 17, 3000, 0, 700, 5000])
 
 
