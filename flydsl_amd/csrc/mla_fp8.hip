@@ -794,26 +794,25 @@ __global__ __launch_bounds__(Shape<NHT>::threads, 1) void mla_fp8_decode_kernel(
   }
 }
 
-// Reductions over the wave: rows of 16 lanes by DPP (quad swaps, then the 8-
-// and 16-lane mirrors), then across the rows.  (Twelve `__shfl_xor` are as many
-// LDS round trips, 0.3 us of a 3.4 us reduce of two pieces.)
+// Reductions over the wave as a butterfly over lanes l ^ 32, 16, 8, 4, 2, 1 (the
+// order of adds of a `__shfl_xor` loop): permlane swaps across the rows of 16
+// lanes, rotations by 8 and 4 (what is rotated has that period by then) and
+// quad swaps within.  Twelve `__shfl_xor` are as many LDS round trips, 0.3 us
+// of a 3.4 us reduce of two pieces.
 template <int CTRL>
 __device__ __forceinline__ float dpp(float v) {
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false));
 }
-__device__ __forceinline__ float wave_max(float v) {
-  v = fmaxf(v, dpp<0xB1>(v));
-  v = fmaxf(v, dpp<0x4E>(v));
-  v = fmaxf(v, dpp<0x141>(v));
-  v = fmaxf(v, dpp<0x140>(v));
-  return max_over_groups(v);
-}
-__device__ __forceinline__ float wave_sum(float v) {
-  v += dpp<0xB1>(v);
-  v += dpp<0x4E>(v);
-  v += dpp<0x141>(v);
-  v += dpp<0x140>(v);
-  return sum_over_groups(v);
+template <typename Op>
+__device__ __forceinline__ float wave_reduce(float v, Op op) {
+  auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  v = op(v, dpp<0x128>(v));
+  v = op(v, dpp<0x124>(v));
+  v = op(v, dpp<0x4E>(v));
+  return op(v, dpp<0xB1>(v));
 }
 
 // One wave per (group, head, 512 / SPLIT value dims): lane l merges 8 / SPLIT
@@ -878,12 +877,12 @@ __global__ __launch_bounds__(256) void mla_fp8_reduce_kernel(const pa_mla_reduce
         }
       };
       load(0);
-      const float mn = fmaxf(mx, wave_max(l));
+      const float mn = fmaxf(mx, wave_reduce(l, [](float x, float y) { return fmaxf(x, y); }));
       const uint64_t live = __ballot(l != kNegInf);
       if (live == 0) continue;
       const float w = l == kNegInf ? 0.f : __expf(l - mn);
       const float fold = mx == kNegInf ? 0.f : __expf(mx - mn);
-      wsum = wsum * fold + wave_sum(w);
+      wsum = wsum * fold + wave_reduce(w, [](float x, float y) { return x + y; });
 #pragma unroll
       for (int j = 0; j < N; ++j) acc[j] *= fold;
       mx = mn;
