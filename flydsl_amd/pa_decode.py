@@ -433,20 +433,23 @@ class _SplitWorkspace:
 _WORKSPACES_KEPT = 16
 _workspaces: "collections.OrderedDict[tuple, _SplitWorkspace]" = collections.OrderedDict()
 _workspaces_lock = threading.Lock()
+_workspace_used = None  # the one used last: already at the end
 
 
 def _native_workspace(index: int, stream_id: int, pairs: int, nbytes: int):
     """Pointers of the workspace of the current stream ``stream_id`` of device
     ``index``, and the workspace itself for the caller to hold."""
+    global _workspace_used
     key = (index, stream_id)
     ws = _workspaces.get(key)
     if ws is None or ws.slots.numel() < nbytes or ws.counters.numel() < pairs:
         ws = _split_workspace(index, torch.cuda.current_stream(index), pairs, nbytes, True)
-    else:
+    elif ws is not _workspace_used:
         try:
             _workspaces.move_to_end(key)
         except KeyError:  # another thread has just dropped it; this call holds it
             pass
+        _workspace_used = ws
     return ws.pointers() + (ws,)
 
 
@@ -459,6 +462,7 @@ def _split_workspace(index: int, stream, pairs: int, nbytes: int, shared: bool):
     dev = torch.device("cuda", index)
     if not shared or sid is None or not (sid == 0 or sid & 1):  # torch's own ids are 0 or odd
         return _SplitWorkspace(dev, stream, nbytes, pairs)
+    global _workspace_used
     key = (index, sid)
     with _workspaces_lock:
         ws = _workspaces.get(key)
@@ -468,6 +472,7 @@ def _split_workspace(index: int, stream, pairs: int, nbytes: int, shared: bool):
             while len(_workspaces) > _WORKSPACES_KEPT:
                 _workspaces.popitem(last=False)
         _workspaces.move_to_end(key)
+        _workspace_used = ws
     return ws
 
 

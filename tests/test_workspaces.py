@@ -21,6 +21,7 @@ class FakeWorkspace:
 def test_the_least_recently_used_workspace_goes(monkeypatch):
     monkeypatch.setattr(pd, "_workspaces", collections.OrderedDict())
     monkeypatch.setattr(pd, "_SplitWorkspace", FakeWorkspace)
+    monkeypatch.setattr(pd, "_workspace_used", None)
     current = SimpleNamespace(stream_id=0)
     monkeypatch.setattr(torch.cuda, "current_stream", lambda index: current)
 
@@ -45,4 +46,5 @@ def test_the_least_recently_used_workspace_goes(monkeypatch):
 
     racing = Racing(pd._workspaces)
     monkeypatch.setattr(pd, "_workspaces", racing)
-    assert use(1) is grown and (0, 1) not in racing
+    last = racing[0, others[-1]]
+    assert use(others[-1]) is last and (0, others[-1]) not in racing
