@@ -2565,7 +2565,7 @@ __global__ __launch_bounds__(64 * WAVES) void pa_fp8_split_kernel(
 // LDS at one workgroup per CU and needs the merge kernel; the slot schedule
 // that such batches took reads them with 8 slots per pair whatever their
 // lengths: 128 sequences of 16 .. 32768 tokens (lognormal), 64 query and 8 kv
-// heads, per-token scales, 204 us -> 126.
+// heads, per-token scales, 204 us -> 124 to 127.
 //
 // The start search costs about 10k cycles (a scan over the batch and three
 // searches), nothing at these sizes.  Cuts: a pair of at most `snap` chunks
@@ -3702,10 +3702,10 @@ __global__ __launch_bounds__(256) void pa_fp8_worklist_reduce8_kernel(const pa_f
 }
 
 // One wave per (sequence, kv head, column); lane l covers head dims 2l,
-// 2l+1.  For each batch of up to 32 slots every load -- the slot's max and
+// 2l+1.  For each batch of up to 16 slots every load -- the slot's max and
 // sum (one slot per lane) and the lane's two values of every slot's partial
 // row -- is issued before any is used, so a row costs one memory round trip
-// per 32 slots; max and sum are then reduced across the wave.
+// per 16 slots; max and sum are then reduced across the wave.
 __global__ __launch_bounds__(256) void pa_fp8_lse_reduce_kernel(const pa_fp8_reduce_args a) {
   constexpr int kBatch = 16;
   const int lane = threadIdx.x & 63;
@@ -4928,13 +4928,15 @@ BalancedLayout balanced_layout(int B, int H, int eq, int nw) {
   return l;
 }
 
+// 16-column blocks up to which the balanced merge runs four columns per wave
+// (the reasons are at its use).
+constexpr int64_t kNarrowMergeBlocks = 512;
+
 // Device scratch of pa_fp8_decode_balanced_static: the balanced split's
 // workspace (pair descriptors, partial lse, partial rows) for callers that
 // cannot allocate.  Each device holds its own copy for the life of the
 // process; the kernels take its device address (kept per device below),
 // never this name, which in host code is only a stand-in.
-// 16-column blocks up to which the balanced merge runs four columns per wave.
-constexpr int64_t kNarrowMergeBlocks = 512;
 constexpr int64_t kStaticScratchBytes = (int64_t)64 << 20;
 static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes];
 
