@@ -13,8 +13,8 @@ which merges them (split decode, one launch); with enough pairs and bounded
 contexts one workgroup per pair (owner launch); batches whose longest
 sequence would set the duration are cut into equal runs of chunks over the
 whole GPU (up to 4 columns: balanced stream split, a decode launch plus a
-merge launch; 5 to 16: team decode, one launch), as are 17 to 64 columns.  Otherwise workgroups take one or a few slots each and
-the reduce kernel merges them.
+merge launch; 5 to 16: team decode, one launch), as are 17 to 64 columns.
+Otherwise workgroups take one or a few slots each and the reduce kernel merges them.
 
 ``exp_sums`` / ``max_logits`` / ``temporary_output`` are workspace, as in
 the reference (preallocated so that graph capture allocates nothing,
